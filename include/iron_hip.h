@@ -396,6 +396,17 @@ int iron_gemm_i4g32_nt(const void* A, const void* codes, const void* scales, voi
                        int splits, void* workspace, long long workspace_bytes, void* stream);
 int iron_gemm_i4g32_splitk_choose(int M, int N, int K);
 
+/* C = clamp(epilogue(A . B)) with B row-major (K, N), read as it is: the
+ * result of iron_gemm_bf16_nt (splits == 1) or iron_gemm_bf16_nt_splitk
+ * (splits > 1, same workspace; NULL otherwise) on the transposed B, bit for
+ * bit, without the transpose. Needs N % 8 == 0, a 16-byte aligned B and
+ * N * K < 2^30 (its byte offsets are 32-bit); everything else as
+ * iron_gemm_bf16_nt. Replaces GEMM with its default row-major B:
+ * iron/operators/gemm/op.py:21-231 (b_col_maj=False). */
+int iron_gemm_bf16_nn(const void* A, const void* B, void* C, int M, int N, int K, long long ldc, int epilogue,
+                      int has_clamp, float clamp_lo, float clamp_hi, int splits, void* workspace,
+                      long long workspace_bytes, void* stream);
+
 /* First pass of the split-K GEMMs alone, for a consumer that merges the
  * partial sums itself (iron_rmsnorm_splitk, iron_qkv_rope_scatter_splitk):
  * workspace (splits, M, N) fp32 receives A . B^T over each of `splits` equal

@@ -5,8 +5,11 @@
 // operands want: with v_mfma_f32_32x32x16_bf16 every lane feeds 8 consecutive
 // k of one row (lane l -> row l%32, k (l/32)*8..+8), so each operand fragment
 // is a single 16-byte LDS read. Other layouts are reduced to this one on the
-// host (B row-major (K, N) through a transpose, C column-major by swapping the
-// operands: C^T = B A^T).
+// host (C column-major by swapping the operands: C^T = B A^T), except a
+// row-major B (K, N) with N % 8 == 0, which the kernel reads as it is (the NN
+// instances, see BRows): its tile is staged k-row by k-row and its fragments
+// come out of LDS through the transposing read ds_read_b64_tr_b16. Any other
+// row-major B goes through a transpose first.
 //
 // Tiles: a workgroup of WMW x WNW waves owns a (WMW*TI*32) x (WNW*TJ*32)
 // output tile; each wave owns TI x TJ MFMA tiles of 32x32. gemm_launch picks
@@ -52,6 +55,7 @@ typedef __bf16 bf16x8_t __attribute__((ext_vector_type(8)));
 typedef float f32x16_t __attribute__((ext_vector_type(16)));
 typedef unsigned int u32x4v __attribute__((ext_vector_type(4)));
 typedef unsigned int u32x2v __attribute__((ext_vector_type(2)));
+typedef short i16x4v __attribute__((ext_vector_type(4)));
 
 constexpr int BK = 64;
 // Buffer offsets are 32-bit: a tile's rows (at most 256) times K times 2 bytes must stay below 2^31.
@@ -316,10 +320,29 @@ __device__ __forceinline__ void tile_coords(const GemmArgs& a, int b, int& kb, i
   tm = t % tiles_m, tn = t / tiles_m;
 }
 
+// B tiles of a row-major B (K, N) (the NN instances): a stage holds BK rows of
+// BN columns, row by row, chunk c (8 columns) of k-row r at slot c ^ swizzle(r).
+// ds_read_b64_tr_b16 serves 32 lanes per LDS pass, here 4 k-rows x 64 bytes; the
+// swizzle puts the four rows' segments on the four quarters of the 64 banks
+// (rows of 128 B already alternate between the two halves). The transpose it
+// replaces read and wrote the whole matrix on every call at ~1.6 TB/s: 2048^3
+// 32.9 -> 23.9 us, the 256-token SwiGLU operator sequence (2048, 8192; three
+// matrices of 33 MB) 160 -> 74 us. The two 8-byte reads per fragment cost
+// what the one 16-byte read of the NT form does.
+template <class T>
+struct BRows {
+  static constexpr int kCols = T::BN / 8;       // 16-byte chunks per k-row
+  static constexpr int kPerBlock = 64 / kCols;  // k-rows per 1 KiB load block
+  static_assert(kCols == 8 || kCols == 16 || kCols == 32, "a k-row must tile 1 KiB blocks");
+  static __device__ __forceinline__ int swizzle(int row) { return kCols == 8 ? ((row >> 1) & 1) << 2 : (row & 3) << 2; }
+};
+
 // TR: the instance launched while a phase trace is armed (trace.hpp); the
 // others carry no trace code. Trace points: 0 start, 1 first stage in LDS,
 // 2-4 after a quarter, half and three quarters of the K steps, 5 tile stored.
-template <class T, bool TR>
+// NN: B is row-major (K, N) instead of (N, K); the MFMA chain is the same, so
+// the result is bit-identical to the NT instance on the transposed matrix.
+template <class T, bool TR, bool NN>
 __global__ __launch_bounds__(T::kThreads) void gemm_nt_kernel(GemmArgs a) {
   constexpr int BM = T::BM, BN = T::BN, TI = T::TI, TJ = T::TJ, NS = T::NS, PW = T::kPerWave;
   __shared__ u32x4v smem[NS * T::kStage];
@@ -340,7 +363,8 @@ __global__ __launch_bounds__(T::kThreads) void gemm_nt_kernel(GemmArgs a) {
   // first A row and first B row (load_lds16). off[j]: byte offset of this lane's
   // chunk at the range's first step.
   const i32x4v rsrc_a = buffer_rsrc(a.A + static_cast<size_t>(m0) * a.K);
-  const i32x4v rsrc_b = buffer_rsrc(a.B + static_cast<size_t>(n0) * a.K);
+  const i32x4v rsrc_b = buffer_rsrc(NN ? a.B : a.B + static_cast<size_t>(n0) * a.K);
+  const unsigned step_b = (NN ? static_cast<unsigned>(a.N) : 1u) * BK * 2;  // bytes from one K step of B to the next
   unsigned off[PW];
 #pragma unroll
   for (int j = 0; j < PW; ++j) {
@@ -350,12 +374,22 @@ __global__ __launch_bounds__(T::kThreads) void gemm_nt_kernel(GemmArgs a) {
     const int chunk = (lane & 7) ^ ((row >> 1) & 7);
     const int r = is_a ? min(m0 + row, a.M - 1) - m0 : min(n0 + row, a.N - 1) - n0;
     off[j] = static_cast<unsigned>((r * a.K + kb * nk * BK + chunk * 8) * 2);
+    if constexpr (NN) {
+      if (!is_a) {  // columns past N load the row's last 8 (N % 8 == 0): they only feed outputs that are never stored
+        using R = BRows<T>;
+        const int kr = (b - BM / 8) * R::kPerBlock + lane / R::kCols;
+        const int col = min(n0 + ((lane % R::kCols) ^ R::swizzle(kr)) * 8, a.N - 8);
+        off[j] = static_cast<unsigned>((kb * nk * BK + kr) * a.N + col) * 2u;
+      }
+    }
   }
   auto issue = [&](int step) {
 #pragma unroll
-    for (int j = 0; j < PW; ++j)
-      load_lds16(wave * PW + j < BM / 8 ? rsrc_a : rsrc_b, off[j] + step * BK * 2,
+    for (int j = 0; j < PW; ++j) {
+      const bool is_a = wave * PW + j < BM / 8;
+      load_lds16(is_a ? rsrc_a : rsrc_b, off[j] + step * (is_a ? BK * 2u : step_b),
                  smem + (step % NS) * T::kStage + (wave * PW + j) * 64);
+    }
   };
 
   f32x16_t acc[TI][TJ];
@@ -366,6 +400,21 @@ __global__ __launch_bounds__(T::kThreads) void gemm_nt_kernel(GemmArgs a) {
 #pragma unroll
       for (int v = 0; v < 16; ++v) acc[i][j][v] = 0.f;
 
+  // NN: this lane's transposed-read address of column block j in a stage's first
+  // k-rows. In each 16-lane group lane 4r + q addresses columns 4q..4q+3 of k-row
+  // r, and lane i receives column i of the four rows; groups 0/1 cover columns 0-15/16-31 of k 0-7, groups 2/3 of k 8-15. k-rows 4
+  // and 16 further on keep the swizzle, so those steps are immediate offsets.
+  unsigned nn_off[TJ];
+  if constexpr (NN) {
+    using R = BRows<T>;
+    const int kr = (lane >> 5) * 8 + ((lane & 15) >> 2);
+#pragma unroll
+    for (int j = 0; j < TJ; ++j) {
+      const int col = (wn * TJ + j) * 32 + ((lane >> 4) & 1) * 16 + (lane & 3) * 4;
+      nn_off[j] = kr * T::BN * 2 + ((col >> 3) ^ R::swizzle(kr)) * 16 + (col & 7) * 2;
+    }
+  }
+
   bf16x8_t fa[2][TI], fb[2][TJ];
   auto read_frags = [&](int set, int stage, int kk) {
     const u32x4v* As = smem + stage * T::kStage;
@@ -374,6 +423,18 @@ __global__ __launch_bounds__(T::kThreads) void gemm_nt_kernel(GemmArgs a) {
 #pragma unroll
     for (int i = 0; i < TI; ++i)
       fa[set][i] = __builtin_bit_cast(bf16x8_t, As[swz(wm * TI * 32 + i * 32 + (lane & 31), c)]);
+    if constexpr (NN) {
+#pragma unroll
+      for (int j = 0; j < TJ; ++j) {
+        const unsigned char* p = reinterpret_cast<const unsigned char*>(Bs) + nn_off[j] + kk * 16 * T::BN * 2;
+        const u32x2v lo = __builtin_bit_cast(
+            u32x2v, __builtin_amdgcn_ds_read_tr16_b64_v4i16((__attribute__((address_space(3))) i16x4v*)(p)));
+        const u32x2v hi = __builtin_bit_cast(
+            u32x2v, __builtin_amdgcn_ds_read_tr16_b64_v4i16((__attribute__((address_space(3))) i16x4v*)(p + 4 * T::BN * 2)));
+        fb[set][j] = __builtin_bit_cast(bf16x8_t, (u32x4v){lo.x, lo.y, hi.x, hi.y});
+      }
+      return;
+    }
 #pragma unroll
     for (int j = 0; j < TJ; ++j)
       fb[set][j] = __builtin_bit_cast(bf16x8_t, Bs[swz(wn * TJ * 32 + j * 32 + (lane & 31), c)]);
@@ -762,14 +823,14 @@ static double launch_cost(const GemmArgs& a, int per_cu, double tflops) {
   return static_cast<double>(rounds * slots) * T::BM * T::BN / tflops;
 }
 
-template <class T>
+template <class T, bool NN>
 static int launch_tile(GemmArgs a, hipStream_t s) {
   const dim3 grid(static_cast<unsigned>(tile_count<T>(a)));
   if (int rc = take_trace("gemm", grid.x, &a.trace)) return rc;
   if (a.trace)
-    IRON_LAUNCH((gemm_nt_kernel<T, true>), grid, dim3(T::kThreads), 0, s, a);
+    IRON_LAUNCH((gemm_nt_kernel<T, true, NN>), grid, dim3(T::kThreads), 0, s, a);
   else
-    IRON_LAUNCH((gemm_nt_kernel<T, false>), grid, dim3(T::kThreads), 0, s, a);
+    IRON_LAUNCH((gemm_nt_kernel<T, false, NN>), grid, dim3(T::kThreads), 0, s, a);
   return 0;
 }
 
@@ -791,30 +852,32 @@ static int small_tile(int M, int N) {
   return 0;
 }
 
+// NN: B is row-major (K, N) (no SwiGLU pair; no 256x192 tiles, whose k-rows do not tile 1 KiB load blocks).
+template <bool NN = false>
 static int gemm_launch(const GemmArgs& a, hipStream_t s) {
   // The SwiGLU pair needs 128-column tiles.
   if (a.splits == 1 && a.epi != kEpiSwigluPair) {
     const int st = small_tile(a.M, a.N);
-    if (st == 64) return launch_tile<Tile64>(a, s);
-    if (st == 128) return launch_tile<Tile128x64>(a, s);
+    if (st == 64) return launch_tile<Tile64, NN>(a, s);
+    if (st == 128) return launch_tile<Tile128x64, NN>(a, s);
   }
   const double cl = launch_cost<TileL>(a, 1, 1000.0), cm = launch_cost<TileM>(a, 1, 900.0);
   const double cs = launch_cost<TileS>(a, 1, 660.0), cs2 = launch_cost<TileS2>(a, 2, 800.0);
   // 256x192 only where it divides N exactly (wave quantization: 3968x3072 gets 256 tiles instead of 192 of
   // 256x256; 72 -> 57 us), and never for the SwiGLU pair epilogue, whose 64-column gate/up blocks must pair
   // up inside a tile.
-  const double cl3 = (a.N % TileL3::BN == 0 && a.epi != kEpiSwigluPair) ? launch_cost<TileL3>(a, 1, 900.0) : 1e300;
+  const double cl3 = (!NN && a.N % TileL3::BN == 0 && a.epi != kEpiSwigluPair) ? launch_cost<TileL3>(a, 1, 900.0) : 1e300;
   const double best = std::min(std::min(std::min(cl, cm), std::min(cs, cs2)), cl3);
-  if (cl3 == best)
-    return launch_tile<TileL3>(a, s);
-  else if (cs == best)
-    return launch_tile<TileS>(a, s);
+  if constexpr (!NN)
+    if (cl3 == best) return launch_tile<TileL3, false>(a, s);
+  if (cs == best)
+    return launch_tile<TileS, NN>(a, s);
   else if (cl == best)
-    return launch_tile<TileL>(a, s);
+    return launch_tile<TileL, NN>(a, s);
   else if (cm == best)
-    return launch_tile<TileM>(a, s);
+    return launch_tile<TileM, NN>(a, s);
   else
-    return launch_tile<TileS2>(a, s);
+    return launch_tile<TileS2, NN>(a, s);
 }
 
 extern "C" int iron_gemm_bf16_nt(const void* A, const void* B, void* C, int M, int N, int K, long long ldc,
@@ -908,6 +971,37 @@ extern "C" int iron_gemm_bf16_nt_splitk(const void* A, const void* B, void* C, i
   if (int rc = gemm_launch(a, s)) return rc;
   launch_splitk_reduce(a, s);
   return check_launch("gemm_bf16_nt_splitk");
+}
+
+// Row-major B: byte offsets into it are 32-bit (from its first element), and
+// its rows are read in 16-byte chunks.
+static bool nn_fits(const void* B, int N, int K) {
+  return N % 8 == 0 && aligned16(B) && static_cast<long long>(N) * K < (1LL << 30);
+}
+
+extern "C" int iron_gemm_bf16_nn(const void* A, const void* B, void* C, int M, int N, int K, long long ldc,
+                                 int epilogue, int has_clamp, float clamp_lo, float clamp_hi, int splits,
+                                 void* workspace, long long workspace_bytes, void* stream) {
+  const char* fn = "iron_gemm_bf16_nn";
+  if (int rc = gemm_check(fn, A, B, C, M, N, K, ldc, epilogue, has_clamp, clamp_lo, clamp_hi)) return rc;
+  IRON_REQUIRE(nn_fits(B, N, K), "%s: a row-major B needs N %% 8 == 0 and N * K < 2^30 (N=%d K=%d)", fn, N, K);
+  IRON_REQUIRE(splits >= 1 && (K / BK) % splits == 0, "%s: splits=%d must divide the %d K steps of 64", fn, splits,
+               K / BK);
+  const long long tiles =
+      static_cast<long long>((M + kSplitTile - 1) / kSplitTile) * ((N + kSplitTile - 1) / kSplitTile) * splits;
+  IRON_REQUIRE(tiles < (1LL << 31) && static_cast<long long>(M) * N < (1LL << 38), "%s: problem too large", fn);
+  if (splits > 1) {
+    const long long need = static_cast<long long>(splits) * M * N * 4;
+    IRON_REQUIRE(workspace && workspace_bytes >= need, "%s: workspace of %lld bytes < %lld", fn, workspace_bytes, need);
+    IRON_REQUIRE(aligned16(workspace), "%s: workspace must be 16-byte aligned", fn);
+  }
+  GemmArgs a{static_cast<const uint16_t*>(A), static_cast<const uint16_t*>(B), static_cast<uint16_t*>(C), M, N, K,
+             ldc, epilogue, has_clamp, clamp_lo, clamp_hi, splits > 1 ? static_cast<float*>(workspace) : nullptr, splits};
+  set_epilogue(a, epilogue);
+  hipStream_t s = static_cast<hipStream_t>(stream);
+  if (int rc = gemm_launch<true>(a, s)) return rc;
+  if (splits > 1) launch_splitk_reduce(a, s);
+  return check_launch("gemm_bf16_nn");
 }
 
 extern "C" int iron_gemm_bf16_nt_swiglu(const void* A, const void* Bgu, void* H, int M, int F, int K, long long ldh,

@@ -4,11 +4,12 @@ Fields and arg spec as the reference: A (M, K); B (K, N), or (N, K) when
 ``b_col_maj``; C (M, N), or (N, M) when ``c_col_maj`` (gemm/reference.py:7-18).
 The AIE tiling knobs are accepted and ignored. K must be a multiple of 64.
 
-Kernel: iron_gemm_bf16_nt (A and B both K-contiguous). B given row-major
-(K, N) is first transposed into an operator-owned scratch buffer; a
-column-major C is produced by computing C^T = B A^T. Shapes whose output
-tiles cannot fill the GPU are split over K (iron_gemm_bf16_nt_splitk, fp32
-partials in an operator-owned workspace).
+Kernels: iron_gemm_bf16_nt (A and B both K-contiguous) and iron_gemm_bf16_nn
+(B row-major (K, N), N a multiple of 8, read as it is). A column-major C is
+produced by computing C^T = B A^T on the former; for that, and for a row-major
+B that the latter does not take, B is first transposed into an operator-owned
+scratch buffer. Shapes whose output tiles cannot fill the GPU are split over K
+(fp32 partials in an operator-owned workspace).
 """
 
 from dataclasses import dataclass, field
@@ -80,16 +81,28 @@ class GEMM(HIPOperator):
         _lib.call("iron_transpose_bf16", B.data_ptr(), bt.data_ptr(), self.K, self.N, stream)
         return bt
 
+    def _splits(self, rows, cols, device):
+        """The K split for rows x cols outputs and its (operator-owned) workspace:
+        (splits, workspace or None, bytes)."""
+        splits = _lib.query("iron_gemm_splitk_choose", rows, cols, self.K)
+        if splits < 2:
+            return 1, None, 0
+        need = int(_lib.query("iron_gemm_splitk_workspace_bytes", rows, cols, splits))
+        ws = self._ws.get(device)
+        if ws is None or ws.numel() < need:
+            ws = torch.empty(need, dtype=torch.uint8, device=device)
+            self._ws[device] = ws
+        return splits, ws, need
+
+    def _nn_takes(self, B) -> bool:
+        """Whether iron_gemm_bf16_nn reads this row-major B (16-byte row chunks, 32-bit byte offsets)."""
+        return self.N % 8 == 0 and self.N * self.K < 1 << 30 and B.data_ptr() % 16 == 0
+
     def _nt(self, X, W, C, rows, cols, stream):
         """C (rows, cols) = X (rows, K) . W (cols, K)^T, split over K when the
-        output tiles alone cannot fill the GPU (operator-owned workspace)."""
-        splits = _lib.query("iron_gemm_splitk_choose", rows, cols, self.K)
+        output tiles alone cannot fill the GPU."""
+        splits, ws, need = self._splits(rows, cols, X.device)
         if splits > 1:
-            need = int(_lib.query("iron_gemm_splitk_workspace_bytes", rows, cols, splits))
-            ws = self._ws.get(X.device)
-            if ws is None or ws.numel() < need:
-                ws = torch.empty(need, dtype=torch.uint8, device=X.device)
-                self._ws[X.device] = ws
             _lib.call("iron_gemm_bf16_nt_splitk", X.data_ptr(), W.data_ptr(), C.data_ptr(), rows, cols, self.K,
                       cols, 0, 0, 0.0, 0.0, splits, ws.data_ptr(), need, stream)
         else:
@@ -97,6 +110,11 @@ class GEMM(HIPOperator):
                       0.0, 0.0, stream)
 
     def _launch(self, A, B, C, *, stream):
+        if not self.b_col_maj and not self.c_col_maj and self._nn_takes(B):
+            splits, ws, need = self._splits(self.M, self.N, A.device)
+            _lib.call("iron_gemm_bf16_nn", A.data_ptr(), B.data_ptr(), C.data_ptr(), self.M, self.N, self.K, self.N, 0,
+                      0, 0.0, 0.0, splits, _lib.ptr(ws), need, stream)
+            return
         Bnk = self._b_nk(B, stream)
         if self.c_col_maj:
             self._nt(Bnk, A, C, self.N, self.M, stream)

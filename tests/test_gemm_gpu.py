@@ -364,3 +364,63 @@ def test_flm_gemm_floor_rounding(gpu, M, K, N, epilogue, clamp):
                    float(rne.reshape(-1)[i])) for i in bad[:5]]
         assert not bad, detail
     assert not bad, bad[:5]
+
+
+# Row-major B (K, N) read as it is: every tile shape, ragged M and N (N % 8 == 0), one and many K steps, a split K.
+@pytest.mark.parametrize(
+    "M,K,N,splits",
+    [
+        (1, 64, 8, 1),  # smallest: one K step, one chunk of columns
+        (100, 320, 200, 1),  # 64x64 tiles, ragged
+        (512, 2048, 3072, 1),  # 128x64 tiles
+        (300, 128, 4104, 1),  # 128x128 tiles of 8 waves, ragged N
+        (1280, 192, 4096, 1),  # 128x128 tiles of 4 waves
+        (2600, 64, 3304, 1),  # 256x128 tiles, ragged
+        (4000, 256, 4104, 1),  # 256x256 tiles, ragged M and N
+        (256, 2048, 2048, 4),  # split K
+        (72, 512, 1000, 2),
+    ],
+)
+@pytest.mark.parametrize("epi", [0, 2])
+def test_gemm_nn_bit_identical_to_nt(gpu, M, K, N, splits, epi):
+    """The MFMA chain of the NN instances is the NT one's, so the results are the same bits."""
+    from iron_amd import _lib
+
+    g = torch.Generator().manual_seed(M + K + N)
+    A = torch.randn(M, K, generator=g).to(BF16).to(gpu)
+    B = (torch.randn(K, N, generator=g) * 0.05).to(BF16).to(gpu)
+    Bt = B.t().contiguous()
+    s = _lib.stream_handle(gpu)
+    ws = torch.empty(splits * M * N, dtype=torch.float32, device=gpu)
+    out = torch.full((M + 1, N), 7.0, dtype=BF16, device=gpu)
+    ref = torch.empty(M, N, dtype=BF16, device=gpu)
+    _lib.call("iron_gemm_bf16_nn", A.data_ptr(), B.data_ptr(), out.data_ptr(), M, N, K, N, epi, 0, 0.0, 0.0, splits,
+              ws.data_ptr(), ws.numel() * 4, s)
+    _lib.call("iron_gemm_bf16_nt_splitk", A.data_ptr(), Bt.data_ptr(), ref.data_ptr(), M, N, K, N, epi, 0, 0.0, 0.0,
+              splits, ws.data_ptr(), ws.numel() * 4, s)
+    torch.cuda.synchronize()
+    assert torch.equal(out[:M], ref)
+    assert (out[M] == 7.0).all()  # nothing past the last row
+
+
+def test_gemm_row_major_b_refused_or_transposed(gpu):
+    """iron_gemm_bf16_nn refuses what it cannot read; the GEMM operator takes those through the transpose."""
+    from iron_amd import _lib
+    from iron_amd.operators import GEMM
+
+    x = torch.zeros(4096, dtype=BF16, device=gpu)
+    for N, off in ((12, 0), (16, 1)):  # rows that are no whole 16-byte chunks; a B that is not 16-byte aligned
+        with pytest.raises(_lib.IronHipError, match="row-major B|16-byte aligned"):
+            _lib.call("iron_gemm_bf16_nn", x.data_ptr(), x.data_ptr() + 2 * off, x.data_ptr(), 4, N, 64, N, 0, 0, 0.0,
+                      0.0, 1, None, 0, _lib.stream_handle(gpu))
+    gen = torch.Generator().manual_seed(5)
+    for N, off in ((203, 0), (200, 1)):
+        A = torch.randn(33, 192, generator=gen).to(BF16)
+        flat = torch.randn(192 * N + off, generator=gen).to(BF16)
+        B = flat[off:].view(192, N)
+        Bd = flat.to(gpu)[off:].view(192, N)
+        C = torch.empty(33, N, dtype=BF16, device=gpu)
+        GEMM(M=33, K=192, N=N).get_callable()(A.to(gpu), Bd, C)
+        torch.cuda.synchronize()
+        ref = A.float() @ B.float()
+        assert ((C.cpu().float() - ref).norm() / ref.norm()) <= 4e-3  # one bf16 rounding is at most 2^-8 of a value
