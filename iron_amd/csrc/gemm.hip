@@ -553,6 +553,14 @@ __device__ __forceinline__ u32x4v dequant8(uint32_t w, float s, bool is_signed) 
   return u32x4v{cvt_pk_bf16(v[0], v[1]), cvt_pk_bf16(v[2], v[3]), cvt_pk_bf16(v[4], v[5]), cvt_pk_bf16(v[6], v[7])};
 }
 
+}  // namespace
+}  // namespace iron
+
+#include "gemm_skinny.hpp"
+
+namespace iron {
+namespace {
+
 template <class T>
 __global__ __launch_bounds__(T::kThreads) void gemm_i4_kernel(GemmArgs a) {
   constexpr int BM = T::BM, BN = T::BN, TI = T::TI, TJ = T::TJ, NS = T::NS, PW = T::kPerWave;
@@ -852,9 +860,62 @@ static int small_tile(int M, int N) {
   return 0;
 }
 
+// Few rows: the streaming kernel of gemm_skinny.hpp instead of the tiles (whose
+// 64 rows would be mostly padding). Cold weights, us before -> after (before:
+// 64x64 / 128x128 tiles with their K split and its merge): 13 x 2048 -> 3072
+// 11.2 -> 4.9, 13 x 8192 -> 2048 15.4 -> 11.1, 13 x 8000 -> 9152 39.6 -> 33.5,
+// 48 x 2048 -> 3072 12.0 -> 7.0, 48 x 2048 -> 8192 18.1 -> 10.5. Past 16 rows a
+// long K goes back to the tiles: a CU takes in ~60 B/ns of cold and L2 data
+// together, and A is then most of it (48 x 8192 -> 2048 16.0 tiled, 18.8 so).
+// The rule sees M and K only: the pair, its two halves and the int4 form of one
+// projection then take the same path, and stay bit-identical.
+static bool skinny(int M, int K) { return M <= 16 || (M <= kSkinnyM && K <= 4096); }
+
+template <int MT, int NT, int KIND, int D>
+static int launch_skinny_tile(GemmArgs a, hipStream_t s) {
+  const int cols = KIND == SK_PAIR ? 16 : 16 * NT, n = KIND == SK_PAIR ? a.N / 2 : a.N;
+  const dim3 grid(static_cast<unsigned>((n + cols - 1) / cols)), block(64 * kSkinnyWaves);
+  if (KIND != SK_I4) {  // the int4 GEMM has no trace points
+    if (int rc = take_trace("gemm", grid.x, &a.trace)) return rc;
+    if (a.trace) {
+      IRON_LAUNCH((gemm_skinny_kernel<MT, NT, KIND, D, true>), grid, block, 0, s, a);
+      return 0;
+    }
+  }
+  IRON_LAUNCH((gemm_skinny_kernel<MT, NT, KIND, D, false>), grid, block, 0, s, a);
+  return 0;
+}
+
+// Two column tiles per workgroup once they still give every CU one (N >= 8192):
+// A is then read half as often. Stages in flight: what the LDS holds, two
+// workgroups per CU where that fits (16 rows; 48 rows with two column tiles).
+template <int KIND>
+static int launch_skinny(const GemmArgs& a, hipStream_t s) {
+  const int mt = (a.M + 15) / 16;
+  if constexpr (KIND == SK_PAIR || KIND == SK_NN) {
+    return mt == 1 ? launch_skinny_tile<1, 2, KIND, 2>(a, s)
+           : mt == 2 ? launch_skinny_tile<2, 2, KIND, 2>(a, s)
+                     : launch_skinny_tile<3, 2, KIND, 1>(a, s);
+  } else {
+    constexpr bool I4 = KIND == SK_I4;
+    const bool wide = a.N >= 8192;
+    if (mt == 1) {
+      if constexpr (I4)
+        if (wide) return launch_skinny_tile<1, 2, KIND, 2>(a, s);
+      return launch_skinny_tile<1, 1, KIND, 2>(a, s);
+    }
+    if (mt == 2) return wide ? launch_skinny_tile<2, 2, KIND, I4 ? 1 : 2>(a, s) : launch_skinny_tile<2, 1, KIND, 2>(a, s);
+    return wide ? launch_skinny_tile<3, 2, KIND, 1>(a, s) : launch_skinny_tile<3, 1, KIND, I4 ? 1 : 2>(a, s);
+  }
+}
+
 // NN: B is row-major (K, N) (no SwiGLU pair; no 256x192 tiles, whose k-rows do not tile 1 KiB load blocks).
 template <bool NN = false>
 static int gemm_launch(const GemmArgs& a, hipStream_t s) {
+  if (a.splits == 1 && !a.partial && skinny(a.M, a.K)) {
+    if constexpr (NN) return launch_skinny<SK_NN>(a, s);
+    return a.epi == kEpiSwigluPair ? launch_skinny<SK_PAIR>(a, s) : launch_skinny<SK_BF16>(a, s);
+  }
   // The SwiGLU pair needs 128-column tiles.
   if (a.splits == 1 && a.epi != kEpiSwigluPair) {
     const int st = small_tile(a.M, a.N);
@@ -925,7 +986,7 @@ static long long plain_small_grid(int M, int N) {
 // at most 512 workgroups (K 8192: M 128 and 256 -> 8 ranges, 512 and 1024 ->
 // 4, 2048 -> 2; 512x8192->2048: 41.7 us plain, 32.1 in 4).
 extern "C" int iron_gemm_splitk_choose(int M, int N, int K) {
-  if (M <= 0 || N <= 0 || K <= 0 || K % BK) return 1;
+  if (M <= 0 || N <= 0 || K <= 0 || K % BK || skinny(M, K)) return 1;
   if (K / BK < 64) return plain_small_grid(M, N) >= 256 ? 1 : splitk_short(M, N, K);
   const long long tiles = static_cast<long long>((M + kSplitTile - 1) / kSplitTile) * ((N + kSplitTile - 1) / kSplitTile);
   int best = 1;
@@ -938,7 +999,7 @@ extern "C" int iron_gemm_splitk_choose(int M, int N, int K) {
 }
 
 extern "C" int iron_gemm_i4g32_splitk_choose(int M, int N, int K) {
-  if (M <= 0 || N <= 0 || K <= 0 || K % BK) return 1;
+  if (M <= 0 || N <= 0 || K <= 0 || K % BK || skinny(M, K)) return 1;
   return splitk_short(M, N, K);
 }
 
@@ -1021,6 +1082,10 @@ extern "C" int iron_gemm_bf16_nt_swiglu(const void* A, const void* Bgu, void* H,
 
 // Cost model for the int4 kernels (measured full-occupancy rates, TFLOP/s).
 static void gemm_i4_launch(const GemmArgs& a, hipStream_t s) {
+  if (a.splits == 1 && !a.partial && skinny(a.M, a.K)) {
+    launch_skinny<SK_I4>(a, s);
+    return;
+  }
   const double cs = launch_cost<TileI4S>(a, 1, 600.0), cm = launch_cost<TileI4M>(a, 1, 800.0);
   if (cs <= cm)
     launch_tile_i4<TileI4S>(a, s);

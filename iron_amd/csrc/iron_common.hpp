@@ -96,6 +96,14 @@ __device__ __forceinline__ void load_lds16(const i32x4v& rsrc, unsigned voffset,
                : "memory", "m0");
 }
 
+// The same with 4 bytes per lane (lane l lands at lds + 4 l).
+__device__ __forceinline__ void load_lds4(const i32x4v& rsrc, unsigned voffset, const void* lds) {
+  const unsigned m0 = __builtin_amdgcn_readfirstlane(static_cast<unsigned>(reinterpret_cast<uintptr_t>(lds)));
+  asm volatile("s_mov_b32 m0, %0\n\ts_nop 0\n\tbuffer_load_dword %1, %2, 0 offen lds" ::"s"(m0), "v"(voffset),
+               "s"(rsrc)
+               : "memory", "m0");
+}
+
 // Argmax key: unsigned order of (value, -index), so the largest key is the
 // largest value and, among equal values, the smallest index.
 __device__ __forceinline__ unsigned long long argmax_key(float v, uint32_t idx) {
