@@ -12,6 +12,7 @@ and torch then share one runtime, one device context and one set of streams.
 from __future__ import annotations
 
 import ctypes
+import functools
 import threading
 from pathlib import Path
 
@@ -131,18 +132,35 @@ def exported_symbols() -> list[str]:
     return ["iron_last_error", "iron_abi_version", *SIGNATURES, *QUERIES]
 
 
+_fns: dict = {}  # entry point name -> its ctypes function, filled on first use
+
+
+def _fn(name: str):
+    fn = _fns.get(name)
+    if fn is None:
+        fn = _fns[name] = getattr(load(), name)
+    return fn
+
+
 def call(name: str, *args) -> None:
     """Invoke entry point ``name``; raise IronHipError with the library's message on failure."""
-    lib = load()
-    rc = getattr(lib, name)(*args)
+    rc = _fn(name)(*args)
     if rc != 0:
-        msg = lib.iron_last_error().decode(errors="replace")
+        msg = load().iron_last_error().decode(errors="replace")
         raise IronHipError(f"{name} failed (code {rc}): {msg}")
 
 
 def query(name: str, *args):
     """Call a value-returning entry point (see QUERIES)."""
-    return getattr(load(), name)(*args)
+    return _fn(name)(*args)
+
+
+@functools.lru_cache(maxsize=4096)
+def gemm_split(policy: str, rows: int, cols: int, K: int) -> tuple[int, int]:
+    """(K ranges, workspace bytes) that the library's split-K ``policy`` query
+    gives a GEMM: a function of the shape alone, so asked once per shape."""
+    splits = int(query(policy, rows, cols, K))
+    return splits, int(query("iron_gemm_splitk_workspace_bytes", rows, cols, splits)) if splits > 1 else 0
 
 
 def ptr(t) -> int | None:
@@ -155,3 +173,11 @@ def stream_handle(device=None) -> int:
     import torch
 
     return torch.cuda.current_stream(device).cuda_stream
+
+
+def tensor_stream(t) -> int:
+    """hipStream_t of torch's current stream on the GPU that holds tensor ``t``
+    (stream_handle(t.device) without building a stream object)."""
+    import torch
+
+    return torch._C._cuda_getCurrentRawStream(t.get_device())

@@ -125,9 +125,8 @@ class GEMM(HIPOperator):
         epi, has_clamp = _EPI_CODE[self.epilogue], int(self.clamp is not None)
         if self.rounding is Rounding.FLOOR:
             epi |= _ROUND_TOWARD_ZERO
-        splits = _lib.query("iron_gemm_splitk_choose", self.M, self.N, self.K)
+        splits, need = _lib.gemm_split("iron_gemm_splitk_choose", self.M, self.N, self.K)
         if splits > 1:  # output tiles alone cannot fill the GPU: split K, merge applies the epilogue
-            need = int(_lib.query("iron_gemm_splitk_workspace_bytes", self.M, self.N, splits))
             ws = self._ws.get(A.device)
             if ws is None or ws.numel() < need:
                 ws = torch.empty(need, dtype=torch.uint8, device=A.device)

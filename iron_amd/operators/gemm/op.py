@@ -84,10 +84,9 @@ class GEMM(HIPOperator):
     def _splits(self, rows, cols, device):
         """The K split for rows x cols outputs and its (operator-owned) workspace:
         (splits, workspace or None, bytes)."""
-        splits = _lib.query("iron_gemm_splitk_choose", rows, cols, self.K)
+        splits, need = _lib.gemm_split("iron_gemm_splitk_choose", rows, cols, self.K)
         if splits < 2:
             return 1, None, 0
-        need = int(_lib.query("iron_gemm_splitk_workspace_bytes", rows, cols, splits))
         ws = self._ws.get(device)
         if ws is None or ws.numel() < need:
             ws = torch.empty(need, dtype=torch.uint8, device=device)

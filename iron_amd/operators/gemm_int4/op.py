@@ -49,10 +49,9 @@ class GEMMInt4(HIPOperator):
         ]
 
     def _launch(self, A, codes, scales, C, *, stream):
-        splits = _lib.query("iron_gemm_i4g32_splitk_choose", self.M, self.N, self.K)
-        ws, need = None, 0
+        splits, need = _lib.gemm_split("iron_gemm_i4g32_splitk_choose", self.M, self.N, self.K)
+        ws = None
         if splits > 1:
-            need = int(_lib.query("iron_gemm_splitk_workspace_bytes", self.M, self.N, splits))
             ws = self._ws.get(A.device)
             if ws is None or ws.numel() < need:
                 ws = torch.empty(need, dtype=torch.uint8, device=A.device)

@@ -18,6 +18,7 @@ The workspace is allocated by the operator (zeroed once) per device.
 
 import math
 from dataclasses import dataclass, field
+from typing import ClassVar
 
 import torch
 
@@ -37,6 +38,8 @@ class GQADecode(HIPOperator):
     context: object = field(default=None, repr=False)
     # bytes of the per-call device phase trace (iron_amd/common/tracing_utils.py); None: IRON_TRACE_SIZE
     trace_size: int | None = field(default=None, repr=False)
+
+    _call_state: ClassVar[frozenset] = frozenset({"position", "position_tensor"})
 
     def __post_init__(self):
         if self.head_dim != 64:
