@@ -378,6 +378,212 @@ __global__ __launch_bounds__(256) void attention_prefill_kernel(PrefillArgs a) {
   }
 }
 
+// ---------------------------------------------------------------------------
+// The same attention where 128-query tiles leave CUs idle (short prompts, or a
+// few new rows behind a long cache): a workgroup owns 32 queries of one head
+// and its W waves split the keys, wave w taking the 32-key blocks w, w + W, ...
+// Each wave streams its blocks through a ring of its own in LDS (two stages of
+// K and V, its own waits, no barrier), with the arithmetic of the kernel above
+// on one S^T tile per block, and the waves' outputs meet once in LDS, rescaled
+// to the common maximum and added in wave order. What bounds the kernel above
+// at these sizes is its serial walk, ~0.9 us per 64 keys on top of ~3.7 us for
+// the launch, the first loads and the output; here the walk is W times shorter
+// (W = 4: 64 KiB of LDS, two workgroups per CU), for K and V read once per 32
+// queries instead of 128. 32/8 heads: 333 rows 9.0 -> 6.2 us, 512 10.8 -> 7.1.
+// ---------------------------------------------------------------------------
+constexpr int kFsK = 32;                   // keys per block
+constexpr int kFsStage = 2 * kFsK * 128;   // a block's K rows, then its V rows (bytes)
+constexpr int kFsDepth = 2;                // stages per wave
+constexpr int kFsStride = 68;              // floats per query of the merge buffer (64 dims, padded)
+
+// W = 8 measured slower than 4 but for a few rows behind a long cache (7 rows
+// behind 3900: 22.9 against 24.7 us; 512 rows 10.2 against 7.1).
+template <int W>
+__global__ __launch_bounds__(64 * W) void attention_prefill_split_kernel(PrefillArgs a) {
+  constexpr int kRing = W * kFsDepth * kFsStage, kMerge = W * 32 * (kFsStride + 2) * 4;
+  __shared__ __attribute__((aligned(16))) unsigned char lds[kRing > kMerge ? kRing : kMerge];
+  const int tid = threadIdx.x, lane = tid & 63;
+  const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
+  const int c = lane & 31, hh = lane >> 5;
+  const int bx = blockIdx.x;  // workgroup order as above: heads that share a KV head on one XCD, longest tiles first
+  const int h = (a.H % 8 == 0) ? (bx % 8) * (a.H / 8) + bx / 8 : bx;
+  const int hk = h / (a.H / a.Hkv);
+  const int tile = a.causal ? static_cast<int>(gridDim.y) - 1 - static_cast<int>(blockIdx.y) : blockIdx.y;
+  const int q0 = tile * 32;
+  if (q0 >= a.Sq) {  // padding rows only (uniform per workgroup)
+    for (int e = tid; e < 32 * (kD / 8); e += 64 * W) {
+      const int r = q0 + (e >> 3), ch = e & 7;
+      if (r < a.out_rows)
+        *reinterpret_cast<fa_u32x4*>(a.out + h * a.o_hs + static_cast<long long>(r) * a.o_rs + ch * 8) =
+            fa_u32x4{0, 0, 0, 0};
+    }
+    return;
+  }
+
+  // Q fragments, consumed before the first K/V load (see the kernel above)
+  fa_bf16x8 qf[4];
+  {
+    const int qrow = min(q0 + c, a.Sq - 1);
+    const uint16_t* qp = a.q + h * a.q_hs + static_cast<long long>(qrow) * a.q_rs;
+#pragma unroll
+    for (int kk = 0; kk < 4; ++kk)
+      qf[kk] = __builtin_bit_cast(fa_bf16x8, *reinterpret_cast<const fa_u32x4*>(qp + 16 * kk + 8 * hh));
+  }
+  asm volatile("" ::"v"(qf[0]), "v"(qf[1]), "v"(qf[2]), "v"(qf[3]));
+  fa_f32x16 o[2];
+#pragma unroll
+  for (int j = 0; j < 16; ++j) o[0][j] = o[1][j] = 0.f;
+  float m = -INFINITY, l = 0.f;
+  const int qpos = a.q_offset + q0 + c;
+  const int first = a.q_offset + q0;  // keys <= it are visible to every query of the tile
+  int kend = a.Skv;
+  if (a.causal) kend = min(kend, a.q_offset + min(q0 + 32, a.Sq));
+  const int nb = (kend + kFsK - 1) / kFsK;
+  const int nw = wave < nb ? (nb - wave + W - 1) / W : 0;  // this wave's blocks
+
+  // Loads 0-3 of a stage are K rows 8 j .. + 7, loads 4-7 the V rows; lane l
+  // lands on row 8 j + l / 8, slot l % 8. Keys past Skv load key Skv - 1.
+  const i32x4v rsrc_k = buffer_rsrc(a.k + hk * a.k_hs), rsrc_v = buffer_rsrc(a.v + hk * a.v_hs);
+  const unsigned krs = static_cast<unsigned>(a.k_rs * 2), vrs = static_cast<unsigned>(a.v_rs * 2);
+  unsigned char* const ring = lds + wave * kFsDepth * kFsStage;
+  auto issue = [&](int i) {
+    unsigned char* st = ring + (i & 1) * kFsStage;
+    const int k0 = (wave + i * W) * kFsK;
+#pragma unroll
+    for (int j = 0; j < 4; ++j) {
+      const int r = j * 8 + (lane >> 3);
+      const unsigned key = static_cast<unsigned>(min(k0 + r, a.Skv - 1));
+      load_lds16(rsrc_k, key * krs + fa_k_slot(r, lane & 7) * 16, st + j * 1024);
+      load_lds16(rsrc_v, key * vrs + fa_v_slot(r, lane & 7) * 16, st + kFsK * 128 + j * 1024);
+    }
+  };
+  static_assert(kFsDepth == 2, "the slots and waits below assume 2 stages of 8 loads");
+  const int tr_row = 4 * hh + ((lane & 15) >> 2), tr_dim = 16 * ((lane >> 4) & 1) + 4 * (lane & 3);
+
+  if (nw > 0) issue(0);
+  if (nw > 1) issue(1);
+  for (int i = 0; i < nw; ++i) {
+    if (i + 1 < nw)
+      asm volatile("s_waitcnt vmcnt(8)" ::: "memory");
+    else
+      asm volatile("s_waitcnt vmcnt(0)" ::: "memory");
+    const unsigned char* ks = ring + (i & 1) * kFsStage;
+    const unsigned char* vs = ks + kFsK * 128;
+    fa_f32x16 sc = {};
+#pragma unroll
+    for (int kk = 0; kk < 4; ++kk) {
+      const fa_bf16x8 kf = __builtin_bit_cast(
+          fa_bf16x8, *reinterpret_cast<const fa_u32x4*>(ks + c * 128 + fa_k_slot(c, 2 * kk + hh) * 16));
+      sc = __builtin_amdgcn_mfma_f32_32x32x16_bf16(kf, qf[kk], sc, 0, 0, 0);
+    }
+    fa_u32x2 vt[2][2][2];
+#pragma unroll
+    for (int db = 0; db < 2; ++db) {
+      const int dim = 32 * db + tr_dim;
+      const unsigned char* vb = vs + tr_row * 128 + fa_v_slot(tr_row, dim >> 3) * 16 + (dim & 7) * 2;
+#pragma unroll
+      for (int st = 0; st < 2; ++st)
+#pragma unroll
+        for (int hl = 0; hl < 2; ++hl)
+          vt[db][st][hl] = __builtin_bit_cast(
+              fa_u32x2, __builtin_amdgcn_ds_read_tr16_b64_v4i16(
+                            (__attribute__((address_space(3))) fa_i16x4*)(vb + 2048 * st + 1024 * hl)));
+    }
+    // online softmax in the log2 domain with lazy rescaling, as above
+    const int k0 = (wave + i * W) * kFsK;
+    const float cs = a.scale_log2;
+    if (k0 + kFsK > a.Skv || (a.causal && k0 + kFsK - 1 > first)) {
+#pragma unroll
+      for (int j = 0; j < 16; ++j) {
+        const int key = k0 + 8 * (j >> 2) + 4 * hh + (j & 3);
+        sc[j] = key < a.Skv && (!a.causal || key <= qpos) ? sc[j] : -INFINITY;
+      }
+    }
+    float mx = fmaxf(fmaxf(sc[0], sc[1]), sc[2]);
+#pragma unroll
+    for (int j = 3; j < 15; j += 2) mx = fmaxf(fmaxf(mx, sc[j]), sc[j + 1]);
+    mx = fa_pair_max(fmaxf(mx, sc[15]));
+    const float mblk = mx * cs;
+    const bool grow = mblk > m + 8.f;
+    if (__builtin_amdgcn_ballot_w64(grow)) {
+      const float alpha = grow ? __builtin_amdgcn_exp2f(m - mblk) : 1.f;  // 0 when m = -inf
+      m = grow ? mblk : m;
+      l *= alpha;
+#pragma unroll
+      for (int j = 0; j < 16; ++j) {
+        o[0][j] *= alpha;
+        o[1][j] *= alpha;
+      }
+    }
+    const float moff = (m == -INFINITY) ? 0.f : m;
+    fa_bf16x8 pf[2];
+#pragma unroll
+    for (int sp = 0; sp < 2; ++sp) {
+      float p[8];
+#pragma unroll
+      for (int e = 0; e < 8; ++e) p[e] = __builtin_amdgcn_exp2f(fmaf(sc[8 * sp + e], cs, -moff));
+      const fa_u32x4 w = {cvt_pk_bf16(p[0], p[1]), cvt_pk_bf16(p[2], p[3]), cvt_pk_bf16(p[4], p[5]),
+                          cvt_pk_bf16(p[6], p[7])};
+#pragma unroll
+      for (int e = 0; e < 4; ++e) l = dot2_bf16(w[e], 0x3f803f80u, l);
+      pf[sp] = __builtin_bit_cast(fa_bf16x8, w);
+    }
+#pragma unroll
+    for (int db = 0; db < 2; ++db)
+#pragma unroll
+      for (int st = 0; st < 2; ++st) {
+        const fa_u32x4 vw = {vt[db][st][0].x, vt[db][st][0].y, vt[db][st][1].x, vt[db][st][1].y};
+        o[db] = __builtin_amdgcn_mfma_f32_32x32x16_bf16(__builtin_bit_cast(fa_bf16x8, vw), pf[st], o[db], 0, 0, 0);
+      }
+    if (i + 2 < nw) {  // every LDS read of this stage has returned before its slot is refilled
+      __builtin_amdgcn_sched_barrier(0);
+      asm volatile("s_waitcnt lgkmcnt(0)" ::: "memory");
+      issue(i + 2);
+    }
+  }
+
+  l = fa_pair_sum(l);
+  __syncthreads();  // every wave is done with its ring
+  float* const mo = reinterpret_cast<float*>(lds);    // [W][32][kFsStride] outputs
+  float* const ml = mo + W * 32 * kFsStride;          // [W][32][2] maximum, sum
+  float* const mine = mo + (wave * 32 + c) * kFsStride;
+#pragma unroll
+  for (int db = 0; db < 2; ++db)
+#pragma unroll
+    for (int j = 0; j < 16; j += 4)
+      *reinterpret_cast<float4*>(mine + 32 * db + 8 * (j >> 2) + 4 * hh) =
+          make_float4(o[db][j], o[db][j + 1], o[db][j + 2], o[db][j + 3]);
+  if (hh == 0) {
+    ml[(wave * 32 + c) * 2] = m;
+    ml[(wave * 32 + c) * 2 + 1] = l;
+  }
+  __syncthreads();
+  for (int e = tid; e < 32 * 8; e += 64 * W) {  // one 8-dim chunk of a query
+    const int r = e >> 3, ch = e & 7, q = q0 + r;
+    float top = -INFINITY;
+#pragma unroll
+    for (int w = 0; w < W; ++w) top = fmaxf(top, ml[(w * 32 + r) * 2]);
+    float sum = 0.f, x[8] = {0.f, 0.f, 0.f, 0.f, 0.f, 0.f, 0.f, 0.f};
+#pragma unroll
+    for (int w = 0; w < W; ++w) {
+      const float mw = ml[(w * 32 + r) * 2];
+      const float f = mw == -INFINITY ? 0.f : __builtin_amdgcn_exp2f(mw - top);  // a wave without visible keys adds nothing
+      sum = fmaf(ml[(w * 32 + r) * 2 + 1], f, sum);
+      const float* p = mo + (w * 32 + r) * kFsStride + ch * 8;
+#pragma unroll
+      for (int d = 0; d < 8; ++d) x[d] = fmaf(p[d], f, x[d]);
+    }
+    const float inv = sum > 0.f ? 1.f / sum : 0.f;
+    uint16_t* dst = a.out + h * a.o_hs + static_cast<long long>(q) * a.o_rs + ch * 8;
+    if (q < a.Sq)
+      *reinterpret_cast<fa_u32x4*>(dst) =
+          fa_u32x4{cvt_pk_bf16(x[0] * inv, x[1] * inv), cvt_pk_bf16(x[2] * inv, x[3] * inv),
+                   cvt_pk_bf16(x[4] * inv, x[5] * inv), cvt_pk_bf16(x[6] * inv, x[7] * inv)};
+    else if (q < a.out_rows)
+      *reinterpret_cast<fa_u32x4*>(dst) = fa_u32x4{0, 0, 0, 0};
+  }
+}
+
 }  // namespace
 }  // namespace iron
 
@@ -678,6 +884,18 @@ extern "C" int iron_attention_prefill(const void* q, const void* k, const void* 
   IRON_REQUIRE(aligned16(out) && o_row_stride % 8 == 0 && o_head_stride % 8 == 0,
                "iron_attention_prefill: out rows must be 16-byte aligned");
   IRON_REQUIRE((out_rows + kFaQ - 1) / kFaQ < 65536, "iron_attention_prefill: out_rows=%d too large", out_rows);
+  // Up to one and a half 128-query tiles per CU the key-split form is faster
+  // (32/8 heads, us, 128-query tiles / split): 128 rows 5.8 / 4.5, 333 9.0 / 6.2,
+  // 512 10.8 / 7.1, 1024 17.7 / 14.8, 1500 (384 tiles) 25.3 / 23.0, 1664 (416)
+  // 26.9 / 27.0, 2048 32.9 / 36.3; 300 rows behind 3600 cached 61.0 / 31.0; at 8/2
+  // heads 2048 rows (128 tiles) 29.9 / 14.2. Past it every CU has work either
+  // way, and K and V read once per 128 queries instead of 32 decide.
+  const long long tiles = static_cast<long long>(n_heads) * ((seq_q + kFaQ - 1) / kFaQ);
+  if (2 * tiles <= 3 * device_cus() && (out_rows + 31) / 32 < 65536) {
+    IRON_LAUNCH((attention_prefill_split_kernel<4>), dim3(n_heads, (out_rows + 31) / 32), dim3(256), 0,
+                static_cast<hipStream_t>(stream), a);
+    return check_launch("attention_prefill");
+  }
   dim3 grid(n_heads, (out_rows + kFaQ - 1) / kFaQ), block(256);
   IRON_LAUNCH(attention_prefill_kernel, grid, block, 0, static_cast<hipStream_t>(stream), a);
   return check_launch("attention_prefill");
