@@ -513,6 +513,13 @@ __global__ __launch_bounds__(T::kThreads) void gemm_nt_kernel(GemmArgs a) {
 // into one of two bf16 tiles (same swizzled layout as a bf16 B stage) after
 // issuing the current step's MFMAs, which read the other tile. The MFMA chain is the bf16 kernel's, so the
 // result is bit-identical to iron_gemm_bf16_nt on the dequantized weights.
+// The next step's codes and scale are read from LDS before the MFMAs and
+// dequantized after them, as plain LDS reads with exact waits (every global
+// load is assembly; with the LDS-direct builtins each such read waited for all
+// loads in flight): 512x2048->8192 33.2 -> 31.5 us, 3968x2048->3072 98 -> 84.
+// What bounds it (same shape, variants): without its loads 24.9 us (the codes'
+// 32-byte and the scales' 4-byte row segments make 384 line requests a step
+// against 256 of the bf16 kernel), without the conversions 28.1.
 // Dequantization: (n ^ 8) (signed) or n via a byte mask, v_cvt_f32_ubyte,
 // one FMA with the scale (q*s = (q+8)*s - 8s exactly), v_cvt_pk_bf16_f32.
 template <int WMW_, int WNW_, int TI_, int TJ_, int NS_>
@@ -583,31 +590,34 @@ __global__ __launch_bounds__(T::kThreads) void gemm_i4_kernel(GemmArgs a) {
 
   // Load slots: A blocks, then code blocks, then scale blocks, then dummies
   // (every wave issues exactly PW loads per step, so one vmcnt count fits all).
-  const unsigned char* src[PW];
+  // All of them are assembly loads (load_lds16, load_lds4): the compiler then
+  // keeps exact counts for the LDS reads below, and can run the dequantization
+  // between the MFMAs. kind is uniform per wave and slot.
+  const i32x4v rsrc_a = buffer_rsrc(a.A + static_cast<size_t>(m0) * a.K);
+  const i32x4v rsrc_c = buffer_rsrc(a.codes + static_cast<size_t>(n0) * (a.K / 2));
+  const i32x4v rsrc_s = buffer_rsrc(a.scales + static_cast<size_t>(n0) * (a.K / 32));
+  unsigned off[PW];
   int dst[PW], kind[PW];  // kind: 0 A (16 B/lane, +128 B per step), 1 codes (16 B, +32 B), 2 scales (4 B, +4 B), 3 dummy
 #pragma unroll
   for (int j = 0; j < PW; ++j) {
     const int slot = wave * PW + j;
     if (slot < T::kABlocks) {
       const int row = slot * 8 + (lane >> 3), chunk = (lane & 7) ^ ((row >> 1) & 7);
-      src[j] = reinterpret_cast<const unsigned char*>(a.A + static_cast<size_t>(min(m0 + row, a.M - 1)) * a.K +
-                                                      static_cast<size_t>(step0) * BK + chunk * 8);
+      off[j] = static_cast<unsigned>((min(m0 + row, a.M - 1) - m0) * a.K + step0 * BK + chunk * 8) * 2u;
       dst[j] = slot * 1024;
       kind[j] = 0;
     } else if (slot < T::kABlocks + T::kCBlocks) {
       const int c = slot - T::kABlocks, row = c * 32 + (lane >> 1);
-      src[j] = a.codes + static_cast<size_t>(min(n0 + row, a.N - 1)) * (a.K / 2) + static_cast<size_t>(step0) * 32 +
-               (lane & 1) * 16;
+      off[j] = static_cast<unsigned>((min(n0 + row, a.N - 1) - n0) * (a.K / 2) + step0 * 32 + (lane & 1) * 16);
       dst[j] = BM * 128 + c * 1024;
       kind[j] = 1;
     } else if (slot < T::kSlots) {
       const int c = slot - T::kABlocks - T::kCBlocks, row = c * 64 + lane;
-      src[j] = reinterpret_cast<const unsigned char*>(a.scales + static_cast<size_t>(min(n0 + row, a.N - 1)) *
-                                                                    (a.K / 32) + static_cast<size_t>(step0) * 2);
+      off[j] = static_cast<unsigned>((min(n0 + row, a.N - 1) - n0) * (a.K / 32) + step0 * 2) * 2u;
       dst[j] = BM * 128 + BN * 32 + c * 256;
       kind[j] = 2;
     } else {
-      src[j] = reinterpret_cast<const unsigned char*>(a.A) + (lane & 7) * 16;  // first 128 B of A (K >= 64)
+      off[j] = (lane & 7) * 16;  // 128 B of the tile's first A row (K >= 64)
       dst[j] = 0;
       kind[j] = 3;
     }
@@ -616,35 +626,34 @@ __global__ __launch_bounds__(T::kThreads) void gemm_i4_kernel(GemmArgs a) {
     unsigned char* st = lds + (step % NS) * T::kStageBytes;
 #pragma unroll
     for (int j = 0; j < PW; ++j) {
-      if (kind[j] == 2)
-        __builtin_amdgcn_global_load_lds(reinterpret_cast<const unsigned*>(src[j] + step * 4),
-                                         reinterpret_cast<unsigned*>(st + dst[j]), 4, 0, 0);
-      else if (kind[j] == 3)
-        __builtin_amdgcn_global_load_lds(reinterpret_cast<const unsigned*>(src[j]),
-                                         reinterpret_cast<unsigned*>(lds + T::kDummyOff), 16, 0, 0);
+      if (kind[j] == 0)
+        load_lds16(rsrc_a, off[j] + step * 128, st + dst[j]);
+      else if (kind[j] == 1)
+        load_lds16(rsrc_c, off[j] + step * 32, st + dst[j]);
+      else if (kind[j] == 2)
+        load_lds4(rsrc_s, off[j] + step * 4, st + dst[j]);
       else
-        __builtin_amdgcn_global_load_lds(reinterpret_cast<const unsigned*>(src[j] + step * (kind[j] == 0 ? 128 : 32)),
-                                         reinterpret_cast<unsigned*>(st + dst[j]), 16, 0, 0);
+        load_lds16(rsrc_a, off[j], lds + T::kDummyOff);
     }
   };
   // Thread -> quarter row of the B tile: row tid / 4, k 16 (tid % 4) .. + 16.
   const int dq_row = tid >> 2, dq_q = tid & 3;
-  // The code and scale reads are inline assembly with their own lgkmcnt wait:
-  // as plain loads, the compiler made them wait vmcnt(0) for every LDS-direct
-  // load in flight (it cannot tell the stages apart).
-  auto dequant = [&](int step) {
-    const unsigned st = static_cast<unsigned>(reinterpret_cast<uintptr_t>(lds)) + (step % NS) * T::kStageBytes;
-    const unsigned ca = st + BM * 128 + dq_row * 32 + dq_q * 8;
-    const unsigned sa = st + BM * 128 + BN * 32 + dq_row * 4 + (dq_q >> 1) * 2;
+  struct Codes {
     u32x2v w;
-    unsigned s16;
-    asm volatile("ds_read_b64 %0, %2\n\tds_read_u16 %1, %3\n\ts_waitcnt lgkmcnt(0)"
-                 : "=&v"(w), "=&v"(s16)
-                 : "v"(ca), "v"(sa));
-    const float sc = __builtin_bit_cast(float, s16 << 16);
+    uint16_t s;
+  };
+  auto read_codes = [&](int step) {
+    const unsigned char* st = lds + (step % NS) * T::kStageBytes;
+    Codes c;
+    c.w = *reinterpret_cast<const u32x2v*>(st + BM * 128 + dq_row * 32 + dq_q * 8);
+    c.s = *reinterpret_cast<const uint16_t*>(st + BM * 128 + BN * 32 + dq_row * 4 + (dq_q >> 1) * 2);
+    return c;
+  };
+  auto dequant = [&](const Codes& c, int step) {
+    const float sc = bf16_to_f32(c.s);
     u32x4v* bt = reinterpret_cast<u32x4v*>(lds + T::kBbfOff + (step & 1) * BN * 128);
-    bt[swz(dq_row, 2 * dq_q)] = dequant8(w.x, sc, a.is_signed);
-    bt[swz(dq_row, 2 * dq_q + 1)] = dequant8(w.y, sc, a.is_signed);
+    bt[swz(dq_row, 2 * dq_q)] = dequant8(c.w.x, sc, a.is_signed);
+    bt[swz(dq_row, 2 * dq_q + 1)] = dequant8(c.w.y, sc, a.is_signed);
   };
 
   f32x16_t acc[TI][TJ];
@@ -663,12 +672,13 @@ __global__ __launch_bounds__(T::kThreads) void gemm_i4_kernel(GemmArgs a) {
     wait_loads_barrier<PW * (NS - 2)>();
   else
     wait_loads_barrier<0>();
-  dequant(0);
+  dequant(read_codes(0), 0);
 
   for (int s = 0; s < nk; ++s) {
+    // This wave's writes of step s's B tile are done (the barrier publishes it).
+    asm volatile("s_waitcnt lgkmcnt(0)" ::: "memory");
     // step s+1 resident (steps s+2..min(s+NS-2, nk-1) may stay in flight); the
-    // barrier also publishes the B tile of step s and retires every read of
-    // the stage and B tile used by step s-1
+    // barrier also retires every read of the stage and B tile used by step s-1
     if (s + NS - 2 < nk)
       wait_loads_barrier<PW * (NS - 3)>();
     else
@@ -687,7 +697,10 @@ __global__ __launch_bounds__(T::kThreads) void gemm_i4_kernel(GemmArgs a) {
         fb[set][j] = __builtin_bit_cast(bf16x8_t, Bs[swz(wn * TJ * 32 + j * 32 + (lane & 31), c)]);
     };
     frags(0, 0);
-    __builtin_amdgcn_iglp_opt(0);  // as in gemm_nt_kernel: 2.6-3.5% faster
+    const Codes next = read_codes(s + 1 < nk ? s + 1 : s);
+    // As in gemm_nt_kernel, for one column tile per wave (512x2048->8192 31.9
+    // -> 31.5 us); with two the compiler's own order is better (3968x2048->3072 84.0 against 86.4).
+    if constexpr (TJ == 1) __builtin_amdgcn_iglp_opt(0);
 #pragma unroll
     for (int kk = 0; kk < BK / 16; ++kk) {
       const int cur = kk & 1, nxt = cur ^ 1;
@@ -698,8 +711,8 @@ __global__ __launch_bounds__(T::kThreads) void gemm_i4_kernel(GemmArgs a) {
         for (int j = 0; j < TJ; ++j)
           acc[i][j] = __builtin_amdgcn_mfma_f32_32x32x16_bf16(fa[cur][i], fb[cur][j], acc[i][j], 0, 0, 0);
     }
-    // the next step's B tile, dequantized while this step's MFMAs execute
-    if (s + 1 < nk) dequant(s + 1);
+    // the next step's B tile; on the last step it repeats this one's into the tile nobody reads any more
+    dequant(next, s + 1);
   }
   store_tile<T>(a, acc, smem, m0, n0, kb, wm, wn, lane, tid);
 }
