@@ -210,16 +210,17 @@ __device__ __forceinline__ void store_tile(const GemmArgs& a, const f32x16_t (&a
   }
   __syncthreads();
   if (swiglu) {
-    // Column blocks 2p and 2p+1 of 64 hold gate and up of features
-    // n0/2 + 64p .. + 63: h = bf16(silu(g) * u) of the bf16-rounded g and u,
+    // Column blocks 2p and 2p+1 of 64 (of 32 in a 64-column tile, see pair_row)
+    // hold gate and up of features n0/2 + 64p .. + 63: h = bf16(silu(g) * u) of the bf16-rounded g and u,
     // as iron_silu_mul on separate gate and up GEMM outputs. C is (M, N/2).
     constexpr int CH = BN / 16;  // 8-feature chunks per output row
+    constexpr int UP = BN == 64 ? 32 : 64;  // columns from gate to up
     const int F = a.N / 2;
     const bool full_f = (n0 / 2 + BN / 2 <= F) && (a.ldc % 8 == 0);
     auto h_chunk = [&](int row, int c) {  // 8 features of one row: silu(g) * u, packed bf16
       const int gcol = (c / 8) * 128 + (c % 8) * 8;
       const uint4 gv = reinterpret_cast<const uint4*>(Cs)[(row * BN + gcol) / 8];
-      const uint4 uv = reinterpret_cast<const uint4*>(Cs)[(row * BN + gcol + 64) / 8];
+      const uint4 uv = reinterpret_cast<const uint4*>(Cs)[(row * BN + gcol + UP) / 8];
       const uint32_t gw[4] = {gv.x, gv.y, gv.z, gv.w}, uw[4] = {uv.x, uv.y, uv.z, uv.w};
       uint32_t h[4];
 #pragma unroll
@@ -242,7 +243,7 @@ __device__ __forceinline__ void store_tile(const GemmArgs& a, const f32x16_t (&a
       const int gm = m0 + row, gf = n0 / 2 + c * 8;
       if (gm >= a.M || gf >= F) continue;
       const uint4 gv = reinterpret_cast<const uint4*>(Cs)[(row * BN + gcol) / 8];
-      const uint4 uv = reinterpret_cast<const uint4*>(Cs)[(row * BN + gcol + 64) / 8];
+      const uint4 uv = reinterpret_cast<const uint4*>(Cs)[(row * BN + gcol + UP) / 8];
       const uint32_t gw[4] = {gv.x, gv.y, gv.z, gv.w}, uw[4] = {uv.x, uv.y, uv.z, uv.w};
       uint32_t h[4];
 #pragma unroll
@@ -320,6 +321,15 @@ __device__ __forceinline__ void tile_coords(const GemmArgs& a, int b, int& kb, i
   tm = t % tiles_m, tn = t / tiles_m;
 }
 
+// Row of B, from the tile's first one, that feeds column r of a SwiGLU pair
+// tile. B alternates 64-row blocks of gate and up, which a tile of 128 or more
+// columns takes as they are; a 64-column tile takes 32 gate rows and the 32 up
+// rows of the same features, 64 rows further on.
+template <class T>
+__device__ __forceinline__ int pair_row(int r) {
+  return T::BN == 64 ? (r & 31) + 64 * (r >> 5) : r;
+}
+
 // B tiles of a row-major B (K, N) (the NN instances): a stage holds BK rows of
 // BN columns, row by row, chunk c (8 columns) of k-row r at slot c ^ swizzle(r).
 // ds_read_b64_tr_b16 serves 32 lanes per LDS pass, here 4 k-rows x 64 bytes; the
@@ -363,7 +373,9 @@ __global__ __launch_bounds__(T::kThreads) void gemm_nt_kernel(GemmArgs a) {
   // first A row and first B row (load_lds16). off[j]: byte offset of this lane's
   // chunk at the range's first step.
   const i32x4v rsrc_a = buffer_rsrc(a.A + static_cast<size_t>(m0) * a.K);
-  const i32x4v rsrc_b = buffer_rsrc(NN ? a.B : a.B + static_cast<size_t>(n0) * a.K);
+  const bool pair64 = BN == 64 && a.epi == kEpiSwigluPair;
+  const int brow0 = pair64 ? (tn >> 1) * 128 + (tn & 1) * 32 : n0;  // the tile's first row of B
+  const i32x4v rsrc_b = buffer_rsrc(NN ? a.B : a.B + static_cast<size_t>(brow0) * a.K);
   const unsigned step_b = (NN ? static_cast<unsigned>(a.N) : 1u) * BK * 2;  // bytes from one K step of B to the next
   unsigned off[PW];
 #pragma unroll
@@ -372,7 +384,8 @@ __global__ __launch_bounds__(T::kThreads) void gemm_nt_kernel(GemmArgs a) {
     const bool is_a = b < BM / 8;
     const int row = (is_a ? b : b - BM / 8) * 8 + (lane >> 3);
     const int chunk = (lane & 7) ^ ((row >> 1) & 7);
-    const int r = is_a ? min(m0 + row, a.M - 1) - m0 : min(n0 + row, a.N - 1) - n0;
+    int r = is_a ? min(m0 + row, a.M - 1) - m0 : min(n0 + row, a.N - 1) - n0;
+    if (pair64 && !is_a) r = pair_row<T>(row);  // N / 2 is a multiple of 64: all inside
     off[j] = static_cast<unsigned>((r * a.K + kb * nk * BK + chunk * 8) * 2);
     if constexpr (NN) {
       if (!is_a) {  // columns past N load the row's last 8 (N % 8 == 0): they only feed outputs that are never stored
@@ -864,7 +877,9 @@ static void launch_tile_i4(const GemmArgs& a, hipStream_t s) {
 // tile whose count comes closest to one per CU without going over (64 = 64x64,
 // 128 = 128x64, 0 = neither fits: the cost model's tiles). 512 tokens, cold
 // weights: 512x2048 -> 2048 19.7 -> 12.3 us (64x64), -> 3072 20.0 -> 15.9 us
-// (128x64), 512x8192 -> 2048 65.6 -> 40.5 us (64x64).
+// (128x64), 512x8192 -> 2048 65.6 -> 40.5 us (64x64). The SwiGLU pair takes them
+// too (pair_row; before, 128x128 tiles on half the CUs): F 8192, K 2048 at 64
+// rows 21.1 -> 16.8 us, 128 rows 24.9 -> 20.5, F 2048, K 2048 at 512 rows 20.3 -> 16.8.
 static int small_tile(int M, int N) {
   auto tiles = [&](int bm, int bn) { return static_cast<long long>((M + bm - 1) / bm) * ((N + bn - 1) / bn); };
   if (tiles(128, 128) >= 256) return 0;
@@ -929,8 +944,7 @@ static int gemm_launch(const GemmArgs& a, hipStream_t s) {
     if constexpr (NN) return launch_skinny<SK_NN>(a, s);
     return a.epi == kEpiSwigluPair ? launch_skinny<SK_PAIR>(a, s) : launch_skinny<SK_BF16>(a, s);
   }
-  // The SwiGLU pair needs 128-column tiles.
-  if (a.splits == 1 && a.epi != kEpiSwigluPair) {
+  if (a.splits == 1) {
     const int st = small_tile(a.M, a.N);
     if (st == 64) return launch_tile<Tile64, NN>(a, s);
     if (st == 128) return launch_tile<Tile128x64, NN>(a, s);

@@ -424,3 +424,28 @@ def test_gemm_row_major_b_refused_or_transposed(gpu):
         torch.cuda.synchronize()
         ref = A.float() @ B.float()
         assert ((C.cpu().float() - ref).norm() / ref.norm()) <= 4e-3  # one bf16 rounding is at most 2^-8 of a value
+
+
+@pytest.mark.parametrize("M,K,F", [(64, 1024, 2048), (49, 8192, 320), (128, 256, 8192), (65, 64, 64), (450, 128, 2112)])
+def test_gemm_swiglu_small_tiles(gpu, M, K, F):
+    """The pair in 64-column tiles (32 gate and 32 up columns each): 64x64 and 128x64 tiles, ragged rows, one K step,
+    an output row stride past F; bit-identical to the two GEMMs and iron_silu_mul."""
+    from iron_amd import _lib
+
+    g = torch.Generator().manual_seed(M + K + F)
+    A = torch.randn(M, K, generator=g).to(BF16).to(gpu)
+    Wg, Wu = ((torch.randn(F, K, generator=g) * 0.05).to(BF16).to(gpu) for _ in range(2))
+    Wgu = _interleave_gate_up(Wg, Wu)
+    s = _lib.stream_handle(gpu)
+    halves = []
+    for W in (Wg, Wu):
+        C = torch.empty(M, F, dtype=BF16, device=gpu)
+        _lib.call("iron_gemm_bf16_nt", A.data_ptr(), W.data_ptr(), C.data_ptr(), M, F, K, F, 0, 0, 0.0, 0.0, s)
+        halves.append(C)
+    ref = torch.empty(M, F, dtype=BF16, device=gpu)
+    _lib.call("iron_silu_mul", halves[0].data_ptr(), halves[1].data_ptr(), ref.data_ptr(), M * F, s)
+    H = torch.full((M + 1, F + 8), 3.0, dtype=BF16, device=gpu)
+    _lib.call("iron_gemm_bf16_nt_swiglu", A.data_ptr(), Wgu.data_ptr(), H.data_ptr(), M, F, K, F + 8, s)
+    torch.cuda.synchronize()
+    assert torch.equal(H[:M, :F], ref)
+    assert (H[:M, F:] == 3.0).all() and (H[M] == 3.0).all()
