@@ -19,8 +19,10 @@ on ROCm), and calls are stream-ordered on torch's current stream.
 
 from __future__ import annotations
 
+import copy
 import dataclasses
 import math
+import operator
 from abc import ABC, abstractmethod
 from dataclasses import dataclass
 from typing import Any, Callable, ClassVar
@@ -140,6 +142,9 @@ def _serialize_param(v: object) -> str:
     return str(v)
 
 
+_PLAIN = frozenset({bool, int, float, str, type(None), torch.dtype})  # types whose values cannot change in place
+
+
 class HIPOperator(AIEOperatorBase):
     """An operator that runs kernels of libiron_hip.so (MLIROperator's role).
 
@@ -150,8 +155,11 @@ class HIPOperator(AIEOperatorBase):
 
     # argument index -> dtypes accepted besides the spec's own
     _extra_dtypes: ClassVar[dict] = {}
-    # attributes that change from call to call and that the arg spec does not depend on
-    _call_state: ClassVar[frozenset] = frozenset()
+    # All that get_arg_spec reads of the operator, as names of plain values (numbers,
+    # texts, dtypes; properties count by value): its specs are then kept between
+    # calls with equal values. Holds for the class that states it, not for subclasses;
+    # without it the specs are built on every call.
+    _spec_fields: ClassVar[tuple[str, ...] | None] = None
     _name_aliases: ClassVar[dict[str, str]] = {
         "num_aie_columns": "c",
         "num_channels": "ch",
@@ -211,31 +219,54 @@ class HIPOperator(AIEOperatorBase):
             if not t.is_contiguous():
                 raise ValueError(f"argument {i} of {type(self).__name__} must be contiguous")
 
-    def __setattr__(self, name: str, value) -> None:
-        object.__setattr__(self, name, value)
-        if name not in self._call_state:
-            self.__dict__.pop("_arg_checks", None)  # the arg spec may have changed
+    def __init_subclass__(cls, **kwargs) -> None:
+        super().__init_subclass__(**kwargs)
+        fields = cls.__dict__.get("_spec_fields")  # its own declaration, not an inherited one
+        cls._spec_values = staticmethod(operator.attrgetter(*fields)) if fields else None
+
+    def _keep_specs(self):
+        """Builds the (dtype, element count) of each argument and keeps them with the
+        values of ``_spec_fields`` they follow from; None for a class that declares
+        none (its spec may depend on anything). Built on a copy, so that another
+        thread that sets a field meanwhile cannot pair one value's spec with another's."""
+        cls = type(self)
+        if cls._spec_values is None or "get_arg_spec" in self.__dict__:
+            return None
+        own = copy.copy(self)
+        key = cls._spec_values(own)
+        if not all(type(v) in _PLAIN for v in (key if isinstance(key, tuple) else (key,))):
+            return None  # a value that could change in place
+        specs = [(s.dtype, s.numel) for s in own.get_arg_spec()]
+        self.__dict__["_spec_kept"] = (key, cls.get_arg_spec, specs)
+        return specs if key == cls._spec_values(self) else None
 
     def _args_fit(self, args) -> bool:
-        """Whether the arguments pass every check of validate_args, without
-        saying which one fails. The specs' dtypes and element counts are kept
-        until an attribute changes: built anew, they and the stream object took
-        ~4 us of a call (int4 GEMV 8192 x 2048 issued back to back 10.2 -> 5.9
-        us a call, GQADecode 16.1 -> 9.9, its kernels 3.2 and 6.5)."""
-        checks = self.__dict__.get("_arg_checks")
-        if checks is None:
-            checks = [((s.dtype, *self._extra_dtypes.get(i, ())), s.numel) for i, s in enumerate(self.get_arg_spec())]
-            self.__dict__["_arg_checks"] = checks
-        if len(args) != len(checks) or not args:
+        """Whether the arguments pass every check of validate_args, without saying
+        which one fails (False also where the specs cannot be kept). Built anew,
+        the specs and the stream object took ~4 us of a call (back to back, int4
+        GEMV 8192 x 2048 10.2 -> 6.1 us a call, GQADecode at 2048 16.5 -> 10.2, their
+        kernels 3.2 and 6.5; ~0.2 of what is left is the comparison of the fields)."""
+        own, cls = self.__dict__, type(self)
+        kept = own.get("_spec_kept")
+        if (kept is not None and kept[0] == cls._spec_values(self) and kept[1] is cls.get_arg_spec
+                and "get_arg_spec" not in own):
+            specs = kept[2]
+        else:
+            specs = self._keep_specs()
+        if specs is None or len(args) != len(specs) or not args:
             return False
         first = args[0]
         if not isinstance(first, torch.Tensor):
             return False
         dev = first.get_device()
-        for t, (dtypes, numel) in zip(args, checks):
-            if not (isinstance(t, torch.Tensor) and t.is_cuda and t.get_device() == dev and t.dtype in dtypes
+        i = 0
+        for t in args:
+            dtype, numel = specs[i]
+            if not (isinstance(t, torch.Tensor) and t.is_cuda and t.get_device() == dev
+                    and (t.dtype is dtype or t.dtype in self._extra_dtypes.get(i, ()))
                     and t.numel() == numel and t.is_contiguous()):
                 return False
+            i += 1
         return True
 
     def get_callable(self) -> Callable[..., Any]:

@@ -12,6 +12,7 @@ nibbles in [-8, 7], the encoding of the fused int4 GEMV weights.
 """
 
 from dataclasses import dataclass, field
+from typing import ClassVar
 
 import torch
 
@@ -30,6 +31,8 @@ class Dequant(HIPOperator):
     group_size: int = field(default=32, repr=False)
     signed: bool = field(default=False, repr=False)
     context: object = field(default=None, repr=False)
+
+    _spec_fields: ClassVar[tuple] = ("input_size", "output_size")
 
     def __post_init__(self):
         self.input_size = (self.size // 2) + (self.size // self.group_size) * 2

@@ -8,4 +8,5 @@ from ..elementwise_mul.op import BinaryElementwise
 
 @dataclass
 class ElementwiseAdd(BinaryElementwise):
+    _spec_fields: ClassVar[tuple] = ("size",)
     _entry: ClassVar[str] = "iron_add"

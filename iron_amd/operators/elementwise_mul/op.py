@@ -39,4 +39,5 @@ class BinaryElementwise(HIPOperator):
 
 @dataclass
 class ElementwiseMul(BinaryElementwise):
+    _spec_fields: ClassVar[tuple] = ("size",)
     _entry: ClassVar[str] = "iron_mul"

@@ -78,6 +78,7 @@ class GEMM(HIPOperator):
         "m_chunk": "mc",
         "rounding": "rnd",
     }
+    _spec_fields: ClassVar[tuple] = ("M", "K", "N")
 
     def __post_init__(self):
         if self.tile_n is None:

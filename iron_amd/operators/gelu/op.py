@@ -8,6 +8,7 @@ reference's GELU); kernel iron_gelu.
 """
 
 from dataclasses import dataclass, field
+from typing import ClassVar
 
 from ... import _lib
 from ...common import HIPOperator, AIERuntimeArgSpec
@@ -20,6 +21,8 @@ class GELU(HIPOperator):
     num_channels: int
     tile_size: int
     context: object = field(default=None, repr=False)
+
+    _spec_fields: ClassVar[tuple] = ("size",)
 
     def __post_init__(self):
         max_multiple = self.num_aie_columns * self.tile_size

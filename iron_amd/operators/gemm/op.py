@@ -51,6 +51,7 @@ class GEMM(HIPOperator):
         "b_col_maj": "bc",
         "c_col_maj": "cc",
     }
+    _spec_fields: ClassVar[tuple] = ("M", "K", "N", "b_col_maj", "c_col_maj")
 
     def __post_init__(self):
         if self.M <= 0 or self.N <= 0 or self.K <= 0:

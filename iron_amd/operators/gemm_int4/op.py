@@ -16,6 +16,7 @@ Shapes whose 128x128 tiles cannot fill the GPU split K into fp32 partials
 """
 
 from dataclasses import dataclass, field
+from typing import ClassVar
 
 import torch
 
@@ -31,6 +32,8 @@ class GEMMInt4(HIPOperator):
     group_size: int = 32
     signed: bool = field(default=True, repr=False)
     context: object = field(default=None, repr=False)
+
+    _spec_fields: ClassVar[tuple] = ("M", "K", "N")
 
     def __post_init__(self):
         if self.group_size != 32:

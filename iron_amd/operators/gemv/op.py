@@ -38,6 +38,7 @@ class GEMV(HIPOperator):
         "tile_size_output": "tso",
         "num_batches": "batch",
     }
+    _spec_fields: ClassVar[tuple] = ("M", "K", "num_batches")
 
     def __post_init__(self):
         if self.tile_size_output is None:

@@ -12,6 +12,7 @@ Arg spec: (codes, scales, vector (K,), output (M,)).
 """
 
 from dataclasses import dataclass, field
+from typing import ClassVar
 
 import torch
 
@@ -28,6 +29,8 @@ class GEMVInt4(HIPOperator):
     context: object = field(default=None, repr=False)
     # bytes of the per-call device phase trace (iron_amd/common/tracing_utils.py); None: IRON_TRACE_SIZE
     trace_size: int | None = field(default=None, repr=False)
+
+    _spec_fields: ClassVar[tuple] = ("M", "K")
 
     def __post_init__(self):
         if self.group_size != 32:

@@ -39,7 +39,7 @@ class GQADecode(HIPOperator):
     # bytes of the per-call device phase trace (iron_amd/common/tracing_utils.py); None: IRON_TRACE_SIZE
     trace_size: int | None = field(default=None, repr=False)
 
-    _call_state: ClassVar[frozenset] = frozenset({"position", "position_tensor"})
+    _spec_fields: ClassVar[tuple] = ("num_heads", "num_kv_heads", "head_dim", "max_len", "angle_rows")
 
     def __post_init__(self):
         if self.head_dim != 64:

@@ -32,6 +32,7 @@ class MHA(HIPOperator):
         "num_KV_heads": "kv",
         "seq_len": "s",
     }
+    _spec_fields: ClassVar[tuple] = ("num_heads", "num_KV_heads", "d", "seq_len", "num_of_pipelines")
 
     def __post_init__(self):
         self.B_q = 64

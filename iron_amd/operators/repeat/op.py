@@ -25,6 +25,7 @@ class Repeat(HIPOperator):
     context: object = field(default=None, repr=False)
 
     _name_aliases: ClassVar[Dict[str, str]] = {**HIPOperator._name_aliases, "repeat": "by", "transfer_size": "ts"}
+    _spec_fields: ClassVar[tuple] = ("rows", "cols", "repeat", "dtype")
 
     def __post_init__(self):
         if self.rows <= 0 or self.cols <= 0 or self.repeat <= 0:

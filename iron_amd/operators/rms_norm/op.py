@@ -29,6 +29,7 @@ class RMSNorm(HIPOperator):
         "weighted": "w",
         "epsilon": "eps",
     }
+    _spec_fields: ClassVar[tuple] = ("rows", "tile_size", "weighted")
 
     def __post_init__(self):
         max_multiple = self.num_aie_columns * self.num_channels * self.tile_size

@@ -33,6 +33,7 @@ class RoPE(HIPOperator):
         "angle_rows": "arows",
         "method_type": "m",
     }
+    _spec_fields: ClassVar[tuple] = ("rows", "cols", "angle_rows")
 
     def __post_init__(self):
         if self.angle_rows is None:

@@ -5,6 +5,7 @@ iron/common/operator_bases.py:22-90; kernel iron_silu.
 """
 
 from dataclasses import dataclass, field
+from typing import ClassVar
 
 from ... import _lib
 from ...common import HIPOperator, AIERuntimeArgSpec
@@ -17,6 +18,8 @@ class SiLU(HIPOperator):
     tile_size: int
     num_channels: int = field(default=1, init=False, repr=False)
     context: object = field(default=None, repr=False)
+
+    _spec_fields: ClassVar[tuple] = ("size",)
 
     def __post_init__(self):
         max_multiple = self.num_aie_columns * self.tile_size

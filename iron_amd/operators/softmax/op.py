@@ -9,6 +9,7 @@ names the runtime parameter that overrides it per call. fp32 math
 """
 
 from dataclasses import dataclass, field
+from typing import ClassVar
 
 from ... import _lib
 from ...common import HIPOperator, AIERuntimeArgSpec
@@ -23,6 +24,8 @@ class Softmax(HIPOperator):
     rtp_vector_size: int | None = None
     vector_size_parameter: str | None = None
     context: object = field(default=None, repr=False)
+
+    _spec_fields: ClassVar[tuple] = ("size",)
 
     @property
     def size(self):

@@ -49,6 +49,7 @@ class StridedCopy(HIPOperator):
         "output_strides": "ost", "output_offset": "ooff", "transfer_size": "tr", "num_aie_channels": "ch",
         "input_offset_parameter": "ipar", "output_offset_parameter": "opar",
     }
+    _spec_fields: ClassVar[tuple] = ("input_buffer_size", "output_buffer_size", "dtype")
 
     def __post_init__(self):
         if len(self.input_sizes) != len(self.input_strides):

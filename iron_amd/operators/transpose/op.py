@@ -27,6 +27,7 @@ class Transpose(HIPOperator):
     context: object = field(default=None, repr=False)
 
     _name_aliases: ClassVar[Dict[str, str]] = {**HIPOperator._name_aliases, "num_batches": "batch"}
+    _spec_fields: ClassVar[tuple] = ("M", "N", "num_batches")
 
     def __post_init__(self):
         if self.M % self.m != 0:
