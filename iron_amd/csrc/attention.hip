@@ -7,6 +7,7 @@
 #include "decode_attn.hpp"
 #include "../../include/iron_hip.h"
 
+#include <algorithm>
 #include <atomic>
 #include <mutex>
 #include <type_traits>
@@ -841,6 +842,34 @@ extern "C" int iron_gqa_decode_noalloc(const void* q, const void* k_new, const v
                            n_heads, n_kv_heads, head_dim, max_len, pos, pos_dev, scale, stream, 0);
 }
 
+// Whether the key-split form takes a call. It always does at up to half a
+// 128-query tile per CU, never past one and a half, nor in between where no walk
+// is longer than 512 keys; else the form with the shorter estimate does (us,
+// above the launch, first loads and output that both pay; fitted to 250 calls,
+// causal or not, 0 to 16000 cached positions, 4 to 64 heads: within 4% of the
+// faster form but for a few). 128-query tiles: the longest tile's walk, 0.86 per
+// 64 keys, and where some CU has two tiles 1.12 per 64 keys of the mean walk.
+// Key split: the workgroups a CU takes in turn, two at a time (0.82 per 128 keys
+// of the mean walk, 2.0 per workgroup), or one walk alone, 0.59 per 128 keys.
+// Us, 128-query tiles / key split, at 32/8 heads: causal, 128 rows 6.2 / 4.9,
+// 512 11.0 / 7.2, 1024 18.1 / 15.4, 1536 26.0 / 24.5; behind 3600 cached, 128
+// rows 53.5 / 21.3, 512 58.6 / 31.1, 1536 89.2 / 90.2; not causal, 512 rows
+// 10.6 / 8.2, 1024 17.9 / 20.0. 64/8 heads, causal: 256 rows 7.9 / 6.2, 640
+// 13.5 / 15.7. 8/2 heads, 4096 rows: causal 56.7 / 35.3, not causal 57.5 / 57.7.
+static bool split_keys(const PrefillArgs& a) {
+  const int cus = device_cus();
+  const long long tiles = static_cast<long long>(a.H) * ((a.Sq + kFaQ - 1) / kFaQ);
+  if (2 * tiles <= cus) return true;
+  if (2 * tiles > 3LL * cus) return false;
+  const double last = a.causal ? std::min<double>(a.Skv, static_cast<double>(a.q_offset) + a.Sq) : a.Skv;
+  const double mean = a.causal ? std::min<double>(a.Skv, a.q_offset + 0.5 * a.Sq) : a.Skv;
+  if (last <= 512) return false;
+  const double turns = static_cast<double>(a.H) * ((a.Sq + 31) / 32) / (2.0 * cus);
+  const double split = std::max(0.59 * last / 128, turns * (0.82 * mean / 128 + 2.0));
+  const double plain = std::max(0.86 * last / 64 + 0.3, tiles > cus ? 1.12 * mean / 64 : 0.0);
+  return split < plain;
+}
+
 extern "C" int iron_attention_prefill(const void* q, const void* k, const void* v, void* out, int n_heads,
                                       int n_kv_heads, int seq_q, int seq_kv, int head_dim, long long q_head_stride,
                                       long long q_row_stride, long long kv_head_stride, long long kv_row_stride,
@@ -884,14 +913,7 @@ extern "C" int iron_attention_prefill(const void* q, const void* k, const void* 
   IRON_REQUIRE(aligned16(out) && o_row_stride % 8 == 0 && o_head_stride % 8 == 0,
                "iron_attention_prefill: out rows must be 16-byte aligned");
   IRON_REQUIRE((out_rows + kFaQ - 1) / kFaQ < 65536, "iron_attention_prefill: out_rows=%d too large", out_rows);
-  // Up to one and a half 128-query tiles per CU the key-split form is faster
-  // (32/8 heads, us, 128-query tiles / split): 128 rows 5.8 / 4.5, 333 9.0 / 6.2,
-  // 512 10.8 / 7.1, 1024 17.7 / 14.8, 1500 (384 tiles) 25.3 / 23.0, 1664 (416)
-  // 26.9 / 27.0, 2048 32.9 / 36.3; 300 rows behind 3600 cached 61.0 / 31.0; at 8/2
-  // heads 2048 rows (128 tiles) 29.9 / 14.2. Past it every CU has work either
-  // way, and K and V read once per 128 queries instead of 32 decide.
-  const long long tiles = static_cast<long long>(n_heads) * ((seq_q + kFaQ - 1) / kFaQ);
-  if (2 * tiles <= 3 * device_cus() && (out_rows + 31) / 32 < 65536) {
+  if (split_keys(a) && (out_rows + 31) / 32 < 65536) {
     IRON_LAUNCH((attention_prefill_split_kernel<4>), dim3(n_heads, (out_rows + 31) / 32), dim3(256), 0,
                 static_cast<hipStream_t>(stream), a);
     return check_launch("attention_prefill");

@@ -51,3 +51,41 @@ def test_prefill_split(gpu, H, Hkv, Sq, Skv, causal, off, pad):
     assert ((out[:, :Sq].double() - ref).abs() <= bound).all()
     assert float((out[:, :Sq].double() - ref).norm() / ref.norm()) <= 6e-3
     assert (out[:, Sq:rows] == 0).all() and (out[:, rows] == 9.0).all()
+
+
+def _attend(q, k, v, causal, off):
+    from iron_amd import _lib
+
+    H, Sq, _ = q.shape
+    Hkv, Skv, _ = k.shape
+    out = torch.empty_like(q)
+    _lib.call("iron_attention_prefill", q.data_ptr(), k.data_ptr(), v.data_ptr(), out.data_ptr(), H, Hkv, Sq, Skv, 64,
+              Sq * 64, 64, Skv * 64, 64, Sq * 64, 64, Sq, causal, off, 0.125, _lib.stream_handle(q.device))
+    return out
+
+
+@pytest.mark.parametrize("H,Hkv,Sq,Skv,causal,off,split", [
+    (64, 8, 640, 640, 1, 0, False),  # 320 query tiles of short walks
+    (64, 8, 384, 384, 1, 0, False),
+    (32, 8, 1024, 1024, 0, 0, False),  # not causal: twice the keys per query
+    (16, 4, 3072, 3072, 0, 0, False),
+    (32, 8, 1536, 17920, 1, 16384, False),  # behind a long cache
+    (64, 8, 256, 256, 0, 0, True),  # half a tile per CU
+    (32, 8, 1024, 1024, 1, 0, True),
+    (32, 8, 768, 4368, 1, 3600, True),
+    (8, 2, 4096, 4096, 1, 0, True),
+])
+def test_form_by_walk(gpu, H, Hkv, Sq, Skv, causal, off, split):
+    """The faster form takes the call. A head's bits say which did: they depend on the form only, the same heads many
+    times over (past one and a half tiles per CU) are in the 128-query form, and one KV group alone (at most half a
+    tile per CU) is in the key-split one."""
+    g = torch.Generator(device=gpu).manual_seed(Sq + Skv)
+    q = torch.randn(H, Sq, 64, device=gpu, generator=g).to(BF16)
+    k, v = (torch.randn(Hkv, Skv, 64, device=gpu, generator=g).to(BF16) for _ in range(2))
+    got, G = _attend(q, k, v, causal, off)[: H // Hkv], H // Hkv
+    times = 2 * 384 // (H * ((Sq + 127) // 128)) + 1
+    whole = _attend(q.repeat(times, 1, 1), k.repeat(times, 1, 1), v.repeat(times, 1, 1), causal, off)[:G]
+    alone = _attend(q[:G].contiguous(), k[:1].contiguous(), v[:1].contiguous(), causal, off)
+    torch.cuda.synchronize()
+    assert not torch.equal(whole, alone)
+    assert torch.equal(got, alone if split else whole)
