@@ -923,21 +923,32 @@ static int small_tile(int M, int N) {
 }
 
 // Few rows: the streaming kernel of gemm_skinny.hpp instead of the tiles (whose
-// 64 rows would be mostly padding). Cold weights, us before -> after (before:
-// 64x64 / 128x128 tiles with their K split and its merge): 13 x 2048 -> 3072
-// 11.2 -> 4.9, 13 x 8192 -> 2048 15.4 -> 11.1, 13 x 8000 -> 9152 39.6 -> 33.5,
-// 48 x 2048 -> 3072 12.0 -> 7.0, 48 x 2048 -> 8192 18.1 -> 10.5. Past 16 rows a
-// long K goes back to the tiles: a CU takes in ~60 B/ns of cold and L2 data
-// together, and A is then most of it (48 x 8192 -> 2048 16.0 tiled, 18.8 so).
-// The rule sees M and K only: the pair, its two halves and the int4 form of one
-// projection then take the same path, and stay bit-identical.
-static bool skinny(int M, int K) { return M <= 16 || (M <= kSkinnyM && K <= 4096); }
+// 64 rows would be mostly padding). Cold weights, us, tiles with their K split
+// and its merge -> this kernel: 13 x 2048 -> 3072 11.5 -> 5.1, 13 x 8192 -> 3072
+// 17.0 -> 12.5, 16 x 4096 -> 16384 38.1 -> 27.1, 48 x 2048 -> 3072 12.2 -> 7.4,
+// 48 x 2048 -> 8192 16.3 -> 10.9; int4 48 x 2048 -> 8192 17.4 -> 7.9.
+// Where the line lies (K 512-4096, N 1024-65536; above it this kernel's time is
+// that of its best column tile): past 16 rows a long K goes back to the tiles,
+// since a CU takes in ~60 B/ns of cold and L2 data together, and A is then most
+// of it (48 x 8192 -> 2048 16.0 tiled, 18.8 so). A wide N does so too, because
+// the launch is then many workgroups per CU, each with an A of its own (48 x 1536
+// -> 16384 12.9 tiled, 14.2 so; 32 x 3072 -> 16384 21.0 and 22.8), but for up to
+// 32 rows whose row pitch is a multiple of 4 KiB, on which the tiles lose more
+// (32 x 4096 -> 16384 38.5 tiled, 28.0 so). The int4 form would gain there (48 x
+// 2048 -> 16384 24.0 tiled, 13.8 so), but keeps the path of the plain one:
+// the rule sees M, K and the columns of the plain product (F of a pair), so that
+// the pair, its two halves, the row-major and the int4 form of one projection
+// stay bit-identical.
+static bool skinny(int M, int N, int K) {
+  if (M <= 16) return true;
+  if (M > kSkinnyM || K > 4096) return false;
+  return N <= 8192 || (M <= 32 && (N <= 10240 || K % 2048 == 0));
+}
 
 template <int MT, int NT, int KIND, int D>
-static int launch_skinny_tile(GemmArgs a, hipStream_t s) {
-  const int cols = KIND == SK_PAIR ? 16 : 16 * NT, n = KIND == SK_PAIR ? a.N / 2 : a.N;
-  const dim3 grid(static_cast<unsigned>((n + cols - 1) / cols)), block(64 * kSkinnyWaves);
-  if (KIND != SK_I4) {  // the int4 GEMM has no trace points
+static int launch_skinny_stages(GemmArgs a, const dim3& grid, hipStream_t s) {
+  const dim3 block(64 * kSkinnyWaves);
+  if constexpr (KIND != SK_I4) {  // the int4 GEMM has no trace points
     if (int rc = take_trace("gemm", grid.x, &a.trace)) return rc;
     if (a.trace) {
       IRON_LAUNCH((gemm_skinny_kernel<MT, NT, KIND, D, true>), grid, block, 0, s, a);
@@ -948,33 +959,51 @@ static int launch_skinny_tile(GemmArgs a, hipStream_t s) {
   return 0;
 }
 
-// Two column tiles per workgroup once they still give every CU one (N >= 8192):
-// A is then read half as often. Stages in flight: what the LDS holds, two
-// workgroups per CU where that fits (16 rows; 48 rows with two column tiles).
+// Two stages in flight per wave where a CU has one workgroup and the LDS holds
+// them; otherwise one, and the CU's other workgroups (as many as fit) cover its
+// waits (two stages / one, us: 16 x 512 -> 65536 22.9 / 15.9, 16 x 768 -> 28672
+// 14.5 / 10.8 in 32 columns; 16 x 1536 -> 16384 11.5 / 11.9 in 64).
+template <int MT, int NT, int KIND>
+static int launch_skinny_tile(const GemmArgs& a, hipStream_t s) {
+  const int cols = KIND == SK_PAIR ? 16 : 16 * NT, n = KIND == SK_PAIR ? a.N / 2 : a.N;
+  const dim3 grid(static_cast<unsigned>((n + cols - 1) / cols));
+  if constexpr (kSkinnyWaves * 2 * SkinnyStage<MT, NT, KIND>::kBytes <= 160 * 1024)
+    if (grid.x <= 256) return launch_skinny_stages<MT, NT, KIND, 2>(a, grid, s);
+  return launch_skinny_stages<MT, NT, KIND, 1>(a, grid, s);
+}
+
+// Columns per workgroup: 16 while that is at most one workgroup per CU, else the
+// 32 or 64 with which a CU takes in fewer rows of A and B (each workgroup reads
+// all of A): 48 x 4096 -> 6144 21.6 us in 16 columns, 16.1 in 32; 32 x 1024 ->
+// 10240 8.4 in 32, 7.7 in 64. The pair's gate and up tile and the row-major
+// form's 64-byte k-rows are 32 columns.
+template <int KIND, int MT>
+static int launch_skinny_rows(const GemmArgs& a, hipStream_t s) {
+  if constexpr (KIND == SK_PAIR || KIND == SK_NN) {
+    return launch_skinny_tile<MT, 2, KIND>(a, s);
+  } else {
+    if (a.N <= 4096) return launch_skinny_tile<MT, 1, KIND>(a, s);
+    if constexpr (MT < 3)  // skinny() takes up to 8192 columns at 33-48 rows
+      if (a.N > 8192) {
+        const long long in2 = (a.N + 8191LL) / 8192 * (MT + 2), in4 = (a.N + 16383LL) / 16384 * (MT + 4);
+        if (in4 < in2) return launch_skinny_tile<MT, 4, KIND>(a, s);
+      }
+    return launch_skinny_tile<MT, 2, KIND>(a, s);
+  }
+}
+
 template <int KIND>
 static int launch_skinny(const GemmArgs& a, hipStream_t s) {
   const int mt = (a.M + 15) / 16;
-  if constexpr (KIND == SK_PAIR || KIND == SK_NN) {
-    return mt == 1 ? launch_skinny_tile<1, 2, KIND, 2>(a, s)
-           : mt == 2 ? launch_skinny_tile<2, 2, KIND, 2>(a, s)
-                     : launch_skinny_tile<3, 2, KIND, 1>(a, s);
-  } else {
-    constexpr bool I4 = KIND == SK_I4;
-    const bool wide = a.N >= 8192;
-    if (mt == 1) {
-      if constexpr (I4)
-        if (wide) return launch_skinny_tile<1, 2, KIND, 2>(a, s);
-      return launch_skinny_tile<1, 1, KIND, 2>(a, s);
-    }
-    if (mt == 2) return wide ? launch_skinny_tile<2, 2, KIND, I4 ? 1 : 2>(a, s) : launch_skinny_tile<2, 1, KIND, 2>(a, s);
-    return wide ? launch_skinny_tile<3, 2, KIND, 1>(a, s) : launch_skinny_tile<3, 1, KIND, I4 ? 1 : 2>(a, s);
-  }
+  return mt == 1   ? launch_skinny_rows<KIND, 1>(a, s)
+         : mt == 2 ? launch_skinny_rows<KIND, 2>(a, s)
+                   : launch_skinny_rows<KIND, 3>(a, s);
 }
 
 // NN: B is row-major (K, N) (no SwiGLU pair; no 256x192 tiles, whose k-rows do not tile 1 KiB load blocks).
 template <bool NN = false>
 static int gemm_launch(const GemmArgs& a, hipStream_t s) {
-  if (a.splits == 1 && !a.partial && skinny(a.M, a.K)) {
+  if (a.splits == 1 && !a.partial && skinny(a.M, a.epi == kEpiSwigluPair ? a.N / 2 : a.N, a.K)) {
     if constexpr (NN) return launch_skinny<SK_NN>(a, s);
     return a.epi == kEpiSwigluPair ? launch_skinny<SK_PAIR>(a, s) : launch_skinny<SK_BF16>(a, s);
   }
@@ -1047,7 +1076,7 @@ static long long plain_small_grid(int M, int N) {
 // at most 512 workgroups (K 8192: M 128 and 256 -> 8 ranges, 512 and 1024 ->
 // 4, 2048 -> 2; 512x8192->2048: 41.7 us plain, 32.1 in 4).
 extern "C" int iron_gemm_splitk_choose(int M, int N, int K) {
-  if (M <= 0 || N <= 0 || K <= 0 || K % BK || skinny(M, K)) return 1;
+  if (M <= 0 || N <= 0 || K <= 0 || K % BK || skinny(M, N, K)) return 1;
   if (K / BK < 64) return plain_small_grid(M, N) >= 256 ? 1 : splitk_short(M, N, K);
   const long long tiles = static_cast<long long>((M + kSplitTile - 1) / kSplitTile) * ((N + kSplitTile - 1) / kSplitTile);
   int best = 1;
@@ -1060,7 +1089,7 @@ extern "C" int iron_gemm_splitk_choose(int M, int N, int K) {
 }
 
 extern "C" int iron_gemm_i4g32_splitk_choose(int M, int N, int K) {
-  if (M <= 0 || N <= 0 || K <= 0 || K % BK || skinny(M, K)) return 1;
+  if (M <= 0 || N <= 0 || K <= 0 || K % BK || skinny(M, N, K)) return 1;
   return splitk_short(M, N, K);
 }
 
@@ -1143,7 +1172,7 @@ extern "C" int iron_gemm_bf16_nt_swiglu(const void* A, const void* Bgu, void* H,
 
 // Cost model for the int4 kernels (measured full-occupancy rates, TFLOP/s).
 static void gemm_i4_launch(const GemmArgs& a, hipStream_t s) {
-  if (a.splits == 1 && !a.partial && skinny(a.M, a.K)) {
+  if (a.splits == 1 && !a.partial && skinny(a.M, a.N, a.K)) {
     launch_skinny<SK_I4>(a, s);
     return;
   }

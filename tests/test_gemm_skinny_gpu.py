@@ -117,3 +117,45 @@ def test_skinny_traced(gpu):
     assert torch.equal(outs[0], outs[1])
     recs = tu.parse_records(buf)
     assert len(recs) == 13 and all(r["name"] == "gemm_bf16" for r in recs)
+
+
+# each width of the column tiles, with one and with two stages in flight, ragged
+@pytest.mark.parametrize("M,K,N", [(16, 192, 8200), (13, 320, 20488), (9, 128, 28680), (17, 320, 8203), (32, 192, 10240),
+                                   (31, 2048, 20488), (20, 2048, 30000), (48, 640, 8192), (40, 64, 4104), (33, 4096, 5001)])
+def test_skinny_column_tiles(gpu, M, K, N):
+    test_skinny_forms(gpu, M, K, N)
+
+
+@pytest.mark.parametrize("M,K,F", [(16, 128, 8192), (20, 192, 5120), (33, 128, 4096), (48, 320, 4160)])
+def test_skinny_pair_stages(gpu, M, K, F):
+    test_skinny_swiglu_pair(gpu, M, K, F)
+
+
+@pytest.mark.parametrize("M,K,N,groups", [
+    (4, 128, 4096, 256),  # 16 columns
+    (48, 4096, 6144, 192),  # 32: one workgroup per CU, not one and a half of 16
+    (16, 512, 20480, 640),
+    (32, 2048, 20480, 640),  # a row pitch of whole 4 KiB
+    (32, 1024, 10240, 160),  # 64
+    (16, 768, 28672, 448),
+    (48, 1536, 16384, 256),  # tiles of 64x64 from here on: wide for their rows
+    (32, 3072, 16384, 256),
+    (33, 64, 8200, 129),
+    (17, 4160, 64, 1),  # a long K
+])
+def test_skinny_range(gpu, M, K, N, groups):
+    """Which kernel takes a call and in how wide columns, by the workgroups of its phase trace: a call goes to the form
+    that is faster for it."""
+    from iron_amd import _lib
+    from iron_amd.common import tracing_utils as tu
+
+    A, _, _, W = _inputs(gpu, M, K, N)
+    C, buf = torch.empty(M, N, dtype=BF16, device=gpu), tu.new_buffer(1 << 17, gpu)
+    tu.arm(buf)
+    _lib.call("iron_gemm_bf16_nt", A.data_ptr(), W.data_ptr(), C.data_ptr(), M, N, K, N, 0, 0, 0.0, 0.0,
+              _lib.stream_handle(gpu))
+    torch.cuda.synchronize()
+    assert len(tu.parse_records(buf)) == groups
+    exact = A.double() @ W.double().t()
+    bound = exact.abs() * 2.0**-8 + K * 2.0**-23 * (A.double().abs() @ W.double().abs().t())
+    assert ((C.double() - exact).abs() <= bound).all()
