@@ -7,8 +7,8 @@ The AIE tiling knobs are accepted and ignored. K must be a multiple of 64.
 Kernels: iron_gemm_bf16_nt (A and B both K-contiguous) and iron_gemm_bf16_nn
 (B row-major (K, N), N a multiple of 8, read as it is). A column-major C is
 produced by computing C^T = B A^T on the former; for that, and for a row-major
-B that the latter does not take, B is first transposed into an operator-owned
-scratch buffer. Shapes whose output tiles cannot fill the GPU are split over K
+B that the latter does not take or is slower on (_nn_takes), B is first
+transposed into an operator-owned scratch buffer. Shapes whose output tiles cannot fill the GPU are split over K
 (fp32 partials in an operator-owned workspace).
 """
 
@@ -95,8 +95,16 @@ class GEMM(HIPOperator):
         return splits, ws, need
 
     def _nn_takes(self, B) -> bool:
-        """Whether iron_gemm_bf16_nn reads this row-major B (16-byte row chunks, 32-bit byte offsets)."""
-        return self.N % 8 == 0 and self.N * self.K < 1 << 30 and B.data_ptr() % 16 == 0
+        """Whether iron_gemm_bf16_nn reads this row-major B (16-byte row chunks, 32-bit
+        byte offsets). A long, narrow B goes through the transpose all the same where
+        the few-row kernel takes the product: its 32-column workgroups are then too
+        few to keep the memory busy, each through all of K (us, as it is / transposed
+        first: 16 x 16384 -> 512 61.4 / 26.3, 16 x 8192 -> 1024 32.5 / 26.5; 16 x 8192
+        -> 256 16.0 / 16.8, 16 x 16384 -> 2048 62.9 / 70.4). The results are the same bits."""
+        M, K, N = self.M, self.K, self.N
+        if M <= 16 and N < 2048 and K >= 8192 and (N * K >= 1 << 22 or K >= 32768):
+            return False
+        return N % 8 == 0 and N * K < 1 << 30 and B.data_ptr() % 16 == 0
 
     def _nt(self, X, W, C, rows, cols, stream):
         """C (rows, cols) = X (rows, K) . W (cols, K)^T, split over K when the

@@ -449,3 +449,29 @@ def test_gemm_swiglu_small_tiles(gpu, M, K, F):
     torch.cuda.synchronize()
     assert torch.equal(H[:M, :F], ref)
     assert (H[:M, F:] == 3.0).all() and (H[M] == 3.0).all()
+
+
+@pytest.mark.parametrize("M,K,N,transposed", [(16, 8192, 512, True), (1, 8256, 1016, True), (16, 32768, 64, True),
+                                              (16, 8192, 256, False), (16, 8192, 2048, False), (16, 8128, 1024, False),
+                                              (17, 8192, 512, False)])
+def test_gemm_few_rows_long_narrow_b(gpu, M, K, N, transposed):
+    """A long, narrow row-major B of a product of few rows goes through the transpose, the faster way to the same bits."""
+    from iron_amd import _lib
+    from iron_amd.operators import GEMM
+
+    g = torch.Generator().manual_seed(K + N)
+    A = torch.randn(M, K, generator=g).to(BF16).to(gpu)
+    B = (torch.randn(K, N, generator=g) * 0.05).to(BF16).to(gpu)
+    op = GEMM(M=M, K=K, N=N)
+    C, ref, out = (torch.empty(M, N, dtype=BF16, device=gpu) for _ in range(3))
+    op.get_callable()(A, B, C)
+    GEMM(M=M, K=K, N=N, b_col_maj=True).get_callable()(A, B.t().contiguous(), ref)
+    torch.cuda.synchronize()
+    assert torch.equal(C, ref)
+    assert bool(op._bt) == transposed
+    splits = _lib.query("iron_gemm_splitk_choose", M, N, K)
+    ws = torch.empty(splits * M * N, dtype=torch.float32, device=gpu)
+    _lib.call("iron_gemm_bf16_nn", A.data_ptr(), B.data_ptr(), out.data_ptr(), M, N, K, N, 0, 0, 0.0, 0.0, splits,
+              ws.data_ptr(), ws.numel() * 4, _lib.stream_handle(gpu))
+    torch.cuda.synchronize()
+    assert torch.equal(out, ref)
