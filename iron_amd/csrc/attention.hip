@@ -382,7 +382,7 @@ __global__ __launch_bounds__(256) void attention_prefill_kernel(PrefillArgs a) {
 // ---------------------------------------------------------------------------
 // The same attention where 128-query tiles leave CUs idle (short prompts, or a
 // few new rows behind a long cache): a workgroup owns 32 queries of one head
-// and its W waves split the keys, wave w taking the 32-key blocks w, w + W, ...
+// and its W = kFsWaves waves split the keys, wave w taking the 32-key blocks w, w + W, ...
 // Each wave streams its blocks through a ring of its own in LDS (two stages of
 // K and V, its own waits, no barrier), with the arithmetic of the kernel above
 // on one S^T tile per block, and the waves' outputs meet once in LDS, rescaled
@@ -397,10 +397,12 @@ constexpr int kFsStage = 2 * kFsK * 128;   // a block's K rows, then its V rows 
 constexpr int kFsDepth = 2;                // stages per wave
 constexpr int kFsStride = 68;              // floats per query of the merge buffer (64 dims, padded)
 
-// W = 8 measured slower than 4 but for a few rows behind a long cache (7 rows
+// 8 measured slower than 4 but for a few rows behind a long cache (7 rows
 // behind 3900: 22.9 against 24.7 us; 512 rows 10.2 against 7.1).
-template <int W>
-__global__ __launch_bounds__(64 * W) void attention_prefill_split_kernel(PrefillArgs a) {
+constexpr int kFsWaves = 4;
+
+__global__ __launch_bounds__(64 * kFsWaves) void attention_prefill_split_kernel(PrefillArgs a) {
+  constexpr int W = kFsWaves;
   constexpr int kRing = W * kFsDepth * kFsStage, kMerge = W * 32 * (kFsStride + 2) * 4;
   __shared__ __attribute__((aligned(16))) unsigned char lds[kRing > kMerge ? kRing : kMerge];
   const int tid = threadIdx.x, lane = tid & 63;
@@ -914,7 +916,7 @@ extern "C" int iron_attention_prefill(const void* q, const void* k, const void* 
                "iron_attention_prefill: out rows must be 16-byte aligned");
   IRON_REQUIRE((out_rows + kFaQ - 1) / kFaQ < 65536, "iron_attention_prefill: out_rows=%d too large", out_rows);
   if (split_keys(a) && (out_rows + 31) / 32 < 65536) {
-    IRON_LAUNCH((attention_prefill_split_kernel<4>), dim3(n_heads, (out_rows + 31) / 32), dim3(256), 0,
+    IRON_LAUNCH(attention_prefill_split_kernel, dim3(n_heads, (out_rows + 31) / 32), dim3(64 * kFsWaves), 0,
                 static_cast<hipStream_t>(stream), a);
     return check_launch("attention_prefill");
   }

@@ -967,9 +967,14 @@ template <int MT, int NT, int KIND>
 static int launch_skinny_tile(const GemmArgs& a, hipStream_t s) {
   const int cols = KIND == SK_PAIR ? 16 : 16 * NT, n = KIND == SK_PAIR ? a.N / 2 : a.N;
   const dim3 grid(static_cast<unsigned>((n + cols - 1) / cols));
-  if constexpr (kSkinnyWaves * 2 * SkinnyStage<MT, NT, KIND>::kBytes <= 160 * 1024)
-    if (grid.x <= 256) return launch_skinny_stages<MT, NT, KIND, 2>(a, grid, s);
-  return launch_skinny_stages<MT, NT, KIND, 1>(a, grid, s);
+  constexpr bool two = kSkinnyWaves * 2 * SkinnyStage<MT, NT, KIND>::kBytes <= 160 * 1024;
+  if constexpr (two && KIND != SK_PAIR && (NT == 1 || MT == 3)) {  // at most 256 workgroups (launch_skinny_rows, skinny)
+    return launch_skinny_stages<MT, NT, KIND, 2>(a, grid, s);
+  } else {
+    if constexpr (two)
+      if (grid.x <= 256) return launch_skinny_stages<MT, NT, KIND, 2>(a, grid, s);
+    return launch_skinny_stages<MT, NT, KIND, 1>(a, grid, s);
+  }
 }
 
 // Columns per workgroup: 16 while that is at most one workgroup per CU, else the

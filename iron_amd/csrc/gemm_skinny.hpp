@@ -4,10 +4,12 @@
 // 0.13 MB of A and C). A workgroup owns 16 * NT output columns and all rows;
 // its 8 waves split K into ranges of whole 128-deep units. Each wave streams
 // the rows of A and B of its range through a ring of its own in LDS
-// (load_lds16: 8 rows x 128 contiguous bytes per instruction) with a few
-// stages in flight, waits for its own loads only and reads the fragments of
-// v_mfma_f32_16x16x32_bf16 from there: no barrier until the waves' fp32 sums
-// meet in LDS, added in wave order. (Fragments loaded straight into registers
+// (load_lds16: 8 rows x 128 contiguous bytes per instruction), waits for its own
+// loads only and reads the fragments of v_mfma_f32_16x16x32_bf16 from there: no
+// barrier until the waves' fp32 sums meet in LDS, added in wave order. One or two
+// stages are in flight per wave (launch_skinny_tile): with one, a stage is loaded
+// once the LDS reads of the one before are done and waited for in full, which the
+// other workgroups of the CU cover. (Fragments loaded straight into registers
 // were limited by the address unit: four adjacent lanes then touch four rows,
 // ~64 clocks per load instead of 16.)
 //
@@ -59,12 +61,13 @@ __device__ __forceinline__ void wait_own_loads() {
 
 // MT: 16-row tiles of M. NT: 16-column tiles (SK_PAIR: tile 0 gate, tile 1 up
 // of the same 16 features; B rows alternate 64-row blocks of gate and up).
-// D: stages in flight per wave. TR: traced instance (points 0 start, 5 stored).
+// D: stages in flight per wave (1 or 2). TR: traced instance (points 0 start, 5 stored).
 template <int MT, int NT, int KIND, int D, bool TR>
 __global__ __launch_bounds__(64 * kSkinnyWaves) void gemm_skinny_kernel(GemmArgs a) {
   using S = SkinnyStage<MT, NT, KIND>;
   constexpr int W = kSkinnyWaves;
   static_assert((KIND != SK_PAIR && KIND != SK_NN) || NT == 2, "a gate and an up tile; 64-byte k-rows");
+  static_assert(D == 1 || D == 2, "the waits of the last stages");
   constexpr int COLS = 16 * NT, ROWS = 16 * MT;
   constexpr int LD = COLS + 1;  // padded row of the reduction buffer
   constexpr int kRing = D * S::kBytes, kRed = W * ROWS * LD * 4;
@@ -224,14 +227,10 @@ __global__ __launch_bounds__(64 * kSkinnyWaves) void gemm_skinny_kernel(GemmArgs
     compute(s);
     issue(s + D);
   }
-  // the last D stages: s1 - s - 1 of them stay in flight
+  // the last D stages
   for (; s < s1; ++s) {
     const int left = s1 - s - 1;
-    if (D > 3 && left >= 3)
-      wait_own_loads<3 * S::kLoads>();
-    else if (D > 2 && left == 2)
-      wait_own_loads<2 * S::kLoads>();
-    else if (D > 1 && left == 1)
+    if (D == 2 && left == 1)
       wait_own_loads<S::kLoads>();
     else
       wait_own_loads<0>();
