@@ -320,15 +320,20 @@ def test_gemm_swiglu_matches_unfused(gpu, M, K, F):
 
 
 @pytest.mark.parametrize("M,K,N,epilogue,clamp", [(256, 512, 1024, "none", None), (256, 512, 1024, "silu", None),
-                                                  (64, 2048, 512, "none", (-50.0, 50.0)), (512, 2048, 2048, "gelu", None)])
+                                                  (64, 2048, 512, "none", (-50.0, 50.0)), (512, 2048, 2048, "gelu", None),
+                                                  (13, 512, 1024, "none", None), (48, 512, 1024, "silu", None),
+                                                  # sums of deviation 418 = sqrt(2048 * 16 * 16 / 3): +-400 leaves about
+                                                  # two thirds unclamped (+-50 one in ten), and half of those truncate
+                                                  # to another value
+                                                  (16, 2048, 512, "none", (-400.0, 400.0)), (1, 1024, 8192, "none", None)])
 def test_flm_gemm_floor_rounding(gpu, M, K, N, epilogue, clamp):
     """flm.GEMM(rounding="floor") (flm/gemm/op.py:105,426-430; the reference's
     test list carries it at 256x512x1024): every output-stage conversion
     truncates. Against the oracle's truncating golden within one bf16 ulp (the
     fp32 sums differ in order, so a value next to a boundary may land one ulp
     apart), and against the same GEMM with round-to-nearest: never larger in
-    magnitude, different in a large share of the elements. The last shape
-    splits K (the merge kernel's conversions)."""
+    magnitude, different in a large share of the elements. 512 rows split K (the
+    merge kernel's conversions), 48 rows and fewer take the few-row kernel."""
     from iron_amd.operators import flm
 
     scale = 4.0 if epilogue == "none" else 0.5
@@ -366,17 +371,17 @@ def test_flm_gemm_floor_rounding(gpu, M, K, N, epilogue, clamp):
     assert not bad, bad[:5]
 
 
-# Row-major B (K, N) read as it is: every tile shape, ragged M and N (N % 8 == 0), one and many K steps, a split K.
+# Row-major B (K, N) read as it is: ragged M and N (N % 8 == 0), one and many K steps, a split K.
 @pytest.mark.parametrize(
     "M,K,N,splits",
     [
-        (1, 64, 8, 1),  # smallest: one K step, one chunk of columns
+        (1, 64, 8, 1),  # smallest: one K step, one chunk of columns (the few-row kernel)
         (100, 320, 200, 1),  # 64x64 tiles, ragged
         (512, 2048, 3072, 1),  # 128x64 tiles
-        (300, 128, 4104, 1),  # 128x128 tiles of 8 waves, ragged N
-        (1280, 192, 4096, 1),  # 128x128 tiles of 4 waves
-        (2600, 64, 3304, 1),  # 256x128 tiles, ragged
-        (4000, 256, 4104, 1),  # 256x256 tiles, ragged M and N
+        (300, 128, 4104, 1),  # 128x64 tiles, ragged N
+        (1280, 192, 4096, 1),  # 256x128 tiles
+        (2600, 64, 3304, 1),  # 256x256 tiles, ragged M and N
+        (4000, 256, 4104, 1),  # 256x128 tiles, ragged M and N
         (256, 2048, 2048, 4),  # split K
         (72, 512, 1000, 2),
     ],
@@ -428,8 +433,9 @@ def test_gemm_row_major_b_refused_or_transposed(gpu):
 
 @pytest.mark.parametrize("M,K,F", [(64, 1024, 2048), (49, 8192, 320), (128, 256, 8192), (65, 64, 64), (450, 128, 2112)])
 def test_gemm_swiglu_small_tiles(gpu, M, K, F):
-    """The pair in 64-column tiles (32 gate and 32 up columns each): 64x64 and 128x64 tiles, ragged rows, one K step,
-    an output row stride past F; bit-identical to the two GEMMs and iron_silu_mul."""
+    """The pair in 64-column tiles (32 gate and 32 up columns each): 64x64 tiles with ragged rows, 128x64 tiles, one
+    K step, an output row stride past F (the last shape takes 128x128 tiles); bit-identical to the two GEMMs and
+    iron_silu_mul."""
     from iron_amd import _lib
 
     g = torch.Generator().manual_seed(M + K + F)
@@ -449,6 +455,66 @@ def test_gemm_swiglu_small_tiles(gpu, M, K, F):
     torch.cuda.synchronize()
     assert torch.equal(H[:M, :F], ref)
     assert (H[:M, F:] == 3.0).all() and (H[M] == 3.0).all()
+
+
+
+def _traced_groups(call):
+    """Workgroups of the GEMM that ``call`` launches, from its phase trace (one record each)."""
+    from iron_amd.common import tracing_utils as tu
+
+    buf = tu.new_buffer(1 << 16, torch.device("cuda", 0))
+    tu.arm(buf)
+    call()
+    torch.cuda.synchronize()
+    return len(tu.parse_records(buf))
+
+
+@pytest.mark.parametrize("M,K,N,groups", [
+    (100, 320, 200, 8),  # 64x64
+    (300, 64, 4104, 195),  # 128x64
+    (300, 64, 8200, 195),  # 128x128 of 8 waves: at most one per CU
+    (640, 64, 12296, 485),  # 128x128 of 4 waves: two per CU
+    (4000, 256, 4104, 528),  # 256x128
+    (2600, 64, 3304, 143),  # 256x256
+])
+def test_gemm_nn_tile_shapes(gpu, M, K, N, groups):
+    """Each tile shape of the row-major form with ragged M and N and stores straight to C; the workgroups of its trace
+    say that the shape is the one meant."""
+    from iron_amd import _lib
+
+    g = torch.Generator().manual_seed(M + K + N)
+    A = torch.randn(M, K, generator=g).to(BF16).to(gpu)
+    B = (torch.randn(K, N, generator=g) * 0.05).to(BF16).to(gpu)
+    s = _lib.stream_handle(gpu)
+    outs = [torch.full((M + 1, N), 7.0, dtype=BF16, device=gpu) for _ in range(2)]
+    run = lambda C: _lib.call("iron_gemm_bf16_nn", A.data_ptr(), B.data_ptr(), C.data_ptr(), M, N, K, N, 0, 0, 0.0, 0.0, 1,
+                              None, 0, s)
+    assert _traced_groups(lambda: run(outs[0])) == groups
+    run(outs[1])  # the instance without a trace
+    torch.cuda.synchronize()
+    exact = A.double() @ B.double()
+    # one bf16 rounding (2^-9 of the value) on top of fp32 sums of K products
+    bound = exact.abs() * 2.0**-8 + K * 2.0**-23 * (A.double().abs() @ B.double().abs())
+    for C in outs:
+        assert ((C[:M].double() - exact).abs() <= bound).all()
+        assert (C[M] == 7.0).all()
+
+
+@pytest.mark.parametrize("M,K,F,groups", [
+    (65, 64, 64, 4),  # 64x64
+    (450, 128, 2048, 256),  # 128x64, ragged rows
+    (450, 128, 2112, 132),  # 128x128
+])
+def test_gemm_swiglu_tile_shapes(gpu, M, K, F, groups):
+    """The pair's tile shapes with ragged rows: the workgroups of its trace, and the bits of the two GEMMs and iron_silu_mul."""
+    from iron_amd import _lib
+
+    A = torch.randn(M, K, generator=torch.Generator().manual_seed(M + F)).to(BF16).to(gpu)
+    W = (torch.randn(2 * F, K, generator=torch.Generator().manual_seed(K)) * 0.05).to(BF16).to(gpu)
+    H = torch.empty(M, F, dtype=BF16, device=gpu)
+    assert _traced_groups(lambda: _lib.call("iron_gemm_bf16_nt_swiglu", A.data_ptr(), W.data_ptr(), H.data_ptr(), M, F, K, F,
+                                            _lib.stream_handle(gpu))) == groups
+    test_gemm_swiglu_small_tiles(gpu, M, K, F)
 
 
 @pytest.mark.parametrize("M,K,N,transposed", [(16, 8192, 512, True), (1, 8256, 1016, True), (16, 32768, 64, True),
