@@ -932,7 +932,8 @@ static int small_tile(int M, int N) {
 // since a CU takes in ~60 B/ns of cold and L2 data together, and A is then most
 // of it (48 x 8192 -> 2048 16.0 tiled, 18.8 so). A wide N does so too, because
 // the launch is then many workgroups per CU, each with an A of its own (48 x 1536
-// -> 16384 12.9 tiled, 14.2 so; 32 x 3072 -> 16384 21.0 and 22.8), but for up to
+// -> 16384 12.9 tiled, 14.2 so; 32 x 3072 -> 16384 21.0 and 22.8; the pair, 26 x
+// 1152 with F 8448, one round of workgroups and a bit, 12.7 and 13.8), but for up to
 // 32 rows whose row pitch is a multiple of 4 KiB, on which the tiles lose more
 // (32 x 4096 -> 16384 38.5 tiled, 28.0 so). The int4 form would gain there (48 x
 // 2048 -> 16384 24.0 tiled, 13.8 so), but keeps the path of the plain one:
@@ -942,7 +943,7 @@ static int small_tile(int M, int N) {
 static bool skinny(int M, int N, int K) {
   if (M <= 16) return true;
   if (M > kSkinnyM || K > 4096) return false;
-  return N <= 8192 || (M <= 32 && (N <= 10240 || K % 2048 == 0));
+  return N <= 8192 || (M <= 32 && K % 2048 == 0);
 }
 
 template <int MT, int NT, int KIND, int D>
@@ -979,8 +980,8 @@ static int launch_skinny_tile(const GemmArgs& a, hipStream_t s) {
 
 // Columns per workgroup: 16 while that is at most one workgroup per CU, else the
 // 32 or 64 with which a CU takes in fewer rows of A and B (each workgroup reads
-// all of A): 48 x 4096 -> 6144 21.6 us in 16 columns, 16.1 in 32; 32 x 1024 ->
-// 10240 8.4 in 32, 7.7 in 64. The pair's gate and up tile and the row-major
+// all of A): 48 x 4096 -> 6144 21.6 us in 16 columns, 16.1 in 32; 32 x 4096 ->
+// 16384 31.2 in 32, 28.0 in 64. The pair's gate and up tile and the row-major
 // form's 64-byte k-rows are 32 columns.
 template <int KIND, int MT>
 static int launch_skinny_rows(const GemmArgs& a, hipStream_t s) {
@@ -988,7 +989,7 @@ static int launch_skinny_rows(const GemmArgs& a, hipStream_t s) {
     return launch_skinny_tile<MT, 2, KIND>(a, s);
   } else {
     if (a.N <= 4096) return launch_skinny_tile<MT, 1, KIND>(a, s);
-    if constexpr (MT < 3)  // skinny() takes up to 8192 columns at 33-48 rows
+    if constexpr (MT < 3)  // skinny() takes at most 8192 columns past 32 rows
       if (a.N > 8192) {
         const long long in2 = (a.N + 8191LL) / 8192 * (MT + 2), in4 = (a.N + 16383LL) / 16384 * (MT + 4);
         if (in4 < in2) return launch_skinny_tile<MT, 4, KIND>(a, s);
