@@ -390,7 +390,7 @@ __global__ __launch_bounds__(256) void attention_prefill_kernel(PrefillArgs a) {
 // at these sizes is its serial walk, ~0.9 us per 64 keys on top of ~3.7 us for
 // the launch, the first loads and the output; here the walk is W times shorter
 // (W = 4: 64 KiB of LDS, two workgroups per CU), for K and V read once per 32
-// queries instead of 128. 32/8 heads: 333 rows 9.0 -> 6.2 us, 512 10.8 -> 7.1.
+// queries instead of 128. 32/8 heads: 333 rows 9.3 -> 6.5 us, 512 11.1 -> 7.2.
 // ---------------------------------------------------------------------------
 constexpr int kFsK = 32;                   // keys per block
 constexpr int kFsStage = 2 * kFsK * 128;   // a block's K rows, then its V rows (bytes)

@@ -200,7 +200,7 @@ __device__ __forceinline__ void store_tile(const GemmArgs& a, const f32x16_t (&a
   // The first rounding to bf16 comes before the activation and the clamp, so
   // those run on the staged tile, where the store reads it back (finish_chunk),
   // with one branch on the activation per tile: tested per accumulator element
-  // they cost 3-18 us (512x2048->8192 silu 26.8 -> 22.9 us, 2509x1920->4096 gelu 74 -> 56).
+  // they cost 3-18 us (512x2048->8192 silu 29.4 -> 26.4 us, 2509x1920->4096 gelu 76 -> 58).
   if (!a.toward_zero) {
 #pragma unroll
     for (int i = 0; i < TI; ++i)
@@ -370,8 +370,8 @@ __device__ __forceinline__ int pair_row(int r) {
 // swizzle puts the four rows' segments on the four quarters of the 64 banks
 // (rows of 128 B already alternate between the two halves). The transpose it
 // replaces read and wrote the whole matrix on every call at ~1.6 TB/s: 2048^3
-// 32.9 -> 23.9 us, the 256-token SwiGLU operator sequence (2048, 8192; three
-// matrices of 33 MB) 160 -> 74 us. The two 8-byte reads per fragment cost
+// 35.7 -> 23.8 us, the 256-token SwiGLU operator sequence (2048, 8192; three
+// matrices of 33 MB) 158 -> 72 us. The two 8-byte reads per fragment cost
 // what the one 16-byte read of the NT form does.
 template <class T>
 struct BRows {
@@ -563,8 +563,9 @@ __global__ __launch_bounds__(T::kThreads) void gemm_nt_kernel(GemmArgs a) {
 // The next step's codes and scale are read from LDS before the MFMAs and
 // dequantized after them, as plain LDS reads with exact waits (every global
 // load is assembly; with the LDS-direct builtins each such read waited for all
-// loads in flight): 512x2048->8192 33.2 -> 31.5 us, 3968x2048->3072 98 -> 84.
-// What bounds it (same shape, variants): without its loads 24.9 us (the codes'
+// loads in flight): 512x2048->8192 29.7 -> 28.1 us, 1000x1024->5120 25.0 -> 21.7,
+// 3968x2048->3072 87 -> 85.
+// What bounds it (first shape, variants, where it took 31.5 us): without its loads 24.9 (the codes'
 // 32-byte and the scales' 4-byte row segments make 384 line requests a step
 // against 256 of the bf16 kernel), without the conversions 28.1.
 // Dequantization: (n ^ 8) (signed) or n via a byte mask, v_cvt_f32_ubyte,
@@ -913,7 +914,7 @@ static void launch_tile_i4(const GemmArgs& a, hipStream_t s) {
 // weights: 512x2048 -> 2048 19.7 -> 12.3 us (64x64), -> 3072 20.0 -> 15.9 us
 // (128x64), 512x8192 -> 2048 65.6 -> 40.5 us (64x64). The SwiGLU pair takes them
 // too (pair_row; before, 128x128 tiles on half the CUs): F 8192, K 2048 at 64
-// rows 21.1 -> 16.8 us, 128 rows 24.9 -> 20.5, F 2048, K 2048 at 512 rows 20.3 -> 16.8.
+// rows 21.6 -> 17.6 us, 128 rows 25.4 -> 20.5, F 2048, K 2048 at 512 rows 20.7 -> 16.9.
 static int small_tile(int M, int N) {
   auto tiles = [&](int bm, int bn) { return static_cast<long long>((M + bm - 1) / bm) * ((N + bn - 1) / bn); };
   if (tiles(128, 128) >= 256) return 0;
