@@ -846,10 +846,10 @@ extern "C" int iron_gqa_decode_noalloc(const void* q, const void* k_new, const v
 
 // Whether the key-split form takes a call. It always does at up to half a
 // 128-query tile per CU, never past one and a half, nor in between where no walk
-// is longer than 512 keys; else the form with the shorter estimate does (us,
-// above the launch, first loads and output that both pay; fitted to 250 calls,
-// causal or not, 0 to 16000 cached positions, 4 to 64 heads: within 4% of the
-// faster form but for a few). 128-query tiles: the longest tile's walk, 0.86 per
+// is longer than 512 keys and there is more than a turn and a quarter of them;
+// else the form with the shorter estimate does (us, above the launch, first
+// loads and output that both pay; fitted to 500 calls, causal or not, 0 to 30000
+// cached positions, 1 to 128 heads: within 5% of the faster form). 128-query tiles: the longest tile's walk, 0.86 per
 // 64 keys, and where some CU has two tiles 1.12 per 64 keys of the mean walk.
 // Key split: the workgroups a CU takes in turn, two at a time (0.82 per 128 keys
 // of the mean walk, 2.0 per workgroup), or one walk alone, 0.59 per 128 keys.
@@ -857,7 +857,7 @@ extern "C" int iron_gqa_decode_noalloc(const void* q, const void* k_new, const v
 // 512 11.0 / 7.2, 1024 18.1 / 15.4, 1536 26.0 / 24.5; behind 3600 cached, 128
 // rows 53.5 / 21.3, 512 58.6 / 31.1, 1536 89.2 / 90.2; not causal, 512 rows
 // 10.6 / 8.2, 1024 17.9 / 20.0. 64/8 heads, causal: 256 rows 7.9 / 6.2, 640
-// 13.5 / 15.7. 8/2 heads, 4096 rows: causal 56.7 / 35.3, not causal 57.5 / 57.7.
+// 13.5 / 15.7; 40/8, 403 rows 9.9 / 8.3. 8/2 heads, 4096 rows: causal 56.7 / 35.3, not causal 57.5 / 57.7.
 static bool split_keys(const PrefillArgs& a) {
   const int cus = device_cus();
   const long long tiles = static_cast<long long>(a.H) * ((a.Sq + kFaQ - 1) / kFaQ);
@@ -865,8 +865,8 @@ static bool split_keys(const PrefillArgs& a) {
   if (2 * tiles > 3LL * cus) return false;
   const double last = a.causal ? std::min<double>(a.Skv, static_cast<double>(a.q_offset) + a.Sq) : a.Skv;
   const double mean = a.causal ? std::min<double>(a.Skv, a.q_offset + 0.5 * a.Sq) : a.Skv;
-  if (last <= 512) return false;
   const double turns = static_cast<double>(a.H) * ((a.Sq + 31) / 32) / (2.0 * cus);
+  if (last <= 512 && turns > 1.25) return false;
   const double split = std::max(0.59 * last / 128, turns * (0.82 * mean / 128 + 2.0));
   const double plain = std::max(0.86 * last / 64 + 0.3, tiles > cus ? 1.12 * mean / 64 : 0.0);
   return split < plain;

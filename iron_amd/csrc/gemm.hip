@@ -933,18 +933,19 @@ static int small_tile(int M, int N) {
 // since a CU takes in ~60 B/ns of cold and L2 data together, and A is then most
 // of it (48 x 8192 -> 2048 16.0 tiled, 18.8 so). A wide N does so too, because
 // the launch is then many workgroups per CU, each with an A of its own (48 x 1536
-// -> 16384 12.9 tiled, 14.2 so; 32 x 3072 -> 16384 21.0 and 22.8; the pair, 26 x
-// 1152 with F 8448, one round of workgroups and a bit, 12.7 and 13.8), but for up to
+// -> 16384 12.9 tiled, 14.2 so; 32 x 3072 -> 16384 21.0 and 22.8), but for up to
 // 32 rows whose row pitch is a multiple of 4 KiB, on which the tiles lose more
-// (32 x 4096 -> 16384 38.5 tiled, 28.0 so). The int4 form would gain there (48 x
-// 2048 -> 16384 24.0 tiled, 13.8 so), but keeps the path of the plain one:
-// the rule sees M, K and the columns of the plain product (F of a pair), so that
-// the pair, its two halves, the row-major and the int4 form of one projection
-// stay bit-identical.
+// (32 x 4096 -> 16384 38.5 tiled, 28.0 so). The rule sees M, K and the columns of
+// the plain product (F of a pair), so that the pair, its two halves, the row-major
+// and the int4 form of one projection take the same path and stay bit-identical.
+// So it weighs them together: over 17-32 rows and 8193-12288 columns the int4 form
+// takes 0.38 of the tiles' time, the plain one 0.84 (at most 1.01), the pair 0.99
+// (0.8 to 1.08, where its workgroups are one round and a bit); over 33-48 rows
+// 0.42 (48 x 2048 -> 16384 24.0 tiled, 13.8 so), 0.91 (to 1.08) and 1.09 (to 1.19).
 static bool skinny(int M, int N, int K) {
   if (M <= 16) return true;
   if (M > kSkinnyM || K > 4096) return false;
-  return N <= 8192 || (M <= 32 && K % 2048 == 0);
+  return N <= 8192 || (M <= 32 && (N <= 12288 || K % 2048 == 0));
 }
 
 template <int MT, int NT, int KIND, int D>

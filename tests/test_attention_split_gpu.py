@@ -71,6 +71,7 @@ def _attend(q, k, v, causal, off):
     (16, 4, 3072, 3072, 0, 0, False),
     (32, 8, 1536, 17920, 1, 16384, False),  # behind a long cache
     (64, 8, 256, 256, 0, 0, True),  # half a tile per CU
+    (40, 8, 403, 403, 1, 0, True),  # short walks, but hardly more than one turn of them
     (32, 8, 1024, 1024, 1, 0, True),
     (32, 8, 768, 4368, 1, 3600, True),
     (8, 2, 4096, 4096, 1, 0, True),

@@ -120,7 +120,7 @@ def test_skinny_traced(gpu):
 
 
 # each width of the column tiles, with one and with two stages in flight, ragged
-@pytest.mark.parametrize("M,K,N", [(16, 192, 8200), (13, 320, 20488), (9, 128, 28680), (17, 2048, 8203), (32, 2048, 10240),
+@pytest.mark.parametrize("M,K,N", [(16, 192, 8200), (13, 320, 20488), (9, 128, 28680), (17, 320, 8203), (32, 192, 10240),
                                    (31, 2048, 20488), (20, 2048, 30000), (48, 640, 8192), (40, 64, 4104), (33, 4096, 5001)])
 def test_skinny_column_tiles(gpu, M, K, N):
     test_skinny_forms(gpu, M, K, N)
@@ -141,6 +141,7 @@ def test_skinny_pair_stages(gpu, M, K, F):
     (48, 1536, 16384, 256),  # tiles of 64x64 from here on: wide for their rows
     (32, 3072, 16384, 256),
     (32, 192, 30000, 235),  # 128x128
+    (32, 1024, 12296, 193),  # 64x64
     (33, 64, 8200, 129),
     (17, 4160, 64, 1),  # a long K
 ])
