@@ -19,7 +19,6 @@ on ROCm), and calls are stream-ordered on torch's current stream.
 
 from __future__ import annotations
 
-import copy
 import dataclasses
 import math
 import operator
@@ -232,7 +231,8 @@ class HIPOperator(AIEOperatorBase):
         cls = type(self)
         if cls._spec_values is None or "get_arg_spec" in self.__dict__:
             return None
-        own = copy.copy(self)
+        own = object.__new__(cls)
+        own.__dict__.update(self.__dict__)
         key = cls._spec_values(own)
         if not all(type(v) in _PLAIN for v in (key if isinstance(key, tuple) else (key,))):
             return None  # a value that could change in place
