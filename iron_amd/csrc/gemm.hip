@@ -962,8 +962,8 @@ static int launch_skinny_stages(GemmArgs a, const dim3& grid, hipStream_t s) {
   return 0;
 }
 
-// Two stages in flight per wave where a CU has one workgroup and the LDS holds
-// them; otherwise one, and the CU's other workgroups (as many as fit) cover its
+// Two stages in flight per wave where a CU has one workgroup (or 16 columns per
+// workgroup) and the LDS holds them; otherwise one, and the CU's other workgroups (as many as fit) cover its
 // waits (two stages / one, us: 16 x 512 -> 65536 22.9 / 15.9, 16 x 768 -> 28672
 // 14.5 / 10.8 in 32 columns; 16 x 1536 -> 16384 11.5 / 11.9 in 64).
 template <int MT, int NT, int KIND>
@@ -971,7 +971,7 @@ static int launch_skinny_tile(const GemmArgs& a, hipStream_t s) {
   const int cols = KIND == SK_PAIR ? 16 : 16 * NT, n = KIND == SK_PAIR ? a.N / 2 : a.N;
   const dim3 grid(static_cast<unsigned>((n + cols - 1) / cols));
   constexpr bool two = kSkinnyWaves * 2 * SkinnyStage<MT, NT, KIND>::kBytes <= 160 * 1024;
-  if constexpr (two && KIND != SK_PAIR && (NT == 1 || MT == 3)) {  // at most 256 workgroups (launch_skinny_rows, skinny)
+  if constexpr (two && KIND != SK_PAIR && (NT == 1 || MT == 3)) {  // 16 columns, or at most 256 workgroups (skinny)
     return launch_skinny_stages<MT, NT, KIND, 2>(a, grid, s);
   } else {
     if constexpr (two)
@@ -983,7 +983,10 @@ static int launch_skinny_tile(const GemmArgs& a, hipStream_t s) {
 // Columns per workgroup: 16 while that is at most one workgroup per CU, else the
 // 32 or 64 with which a CU takes in fewer rows of A and B (each workgroup reads
 // all of A): 48 x 4096 -> 6144 21.6 us in 16 columns, 16.1 in 32; 32 x 4096 ->
-// 16384 31.2 in 32, 28.0 in 64. The pair's gate and up tile and the row-major
+// 16384 31.2 in 32, 28.0 in 64. But 16 again for a long K of up to 8 bf16 rows,
+// whose A costs little (rows past M repeat the last one: 4 x 3072 -> 20480 23.4, 26.2
+// in 32), and for up to 16 at a row pitch of 4 KiB (16 x 2048 -> 12288 11.6, 13.4 in
+// 64; 16 x 3072 -> 12288 17.2 and 16.9, 16 x 4608 -> 14336 29.6 and 26.1). The pair's gate and up tile and the row-major
 // form's 64-byte k-rows are 32 columns.
 template <int KIND, int MT>
 static int launch_skinny_rows(const GemmArgs& a, hipStream_t s) {
@@ -991,6 +994,9 @@ static int launch_skinny_rows(const GemmArgs& a, hipStream_t s) {
     return launch_skinny_tile<MT, 2, KIND>(a, s);
   } else {
     if (a.N <= 4096) return launch_skinny_tile<MT, 1, KIND>(a, s);
+    if constexpr (MT == 1 && KIND == SK_BF16)
+      if (a.N > 8192 && a.K >= 2048 && (a.M <= 8 || a.K == 2048))
+        return launch_skinny_tile<MT, 1, KIND>(a, s);
     if constexpr (MT < 3)  // skinny() takes at most 8192 columns past 32 rows
       if (a.N > 8192) {
         const long long in2 = (a.N + 8191LL) / 8192 * (MT + 2), in4 = (a.N + 16383LL) / 16384 * (MT + 4);

@@ -121,7 +121,7 @@ def test_skinny_traced(gpu):
 
 # each width of the column tiles, with one and with two stages in flight, ragged
 @pytest.mark.parametrize("M,K,N", [(16, 192, 8200), (13, 320, 20488), (9, 128, 28680), (17, 320, 8203), (32, 192, 10240),
-                                   (31, 2048, 20488), (20, 2048, 30000), (48, 640, 8192), (40, 64, 4104), (33, 4096, 5001)])
+                                   (31, 2048, 20488), (20, 2048, 30000), (48, 640, 8192), (40, 64, 4104), (33, 4096, 5001), (9, 2048, 8200)])
 def test_skinny_column_tiles(gpu, M, K, N):
     test_skinny_forms(gpu, M, K, N)
 
@@ -136,6 +136,9 @@ def test_skinny_pair_stages(gpu, M, K, F):
     (48, 4096, 6144, 192),  # 32: one workgroup per CU, not one and a half of 16
     (16, 512, 20480, 640),
     (32, 2048, 20480, 640),  # a row pitch of whole 4 KiB
+    (8, 2112, 16384, 1024),  # 16 again: a long K of few rows
+    (13, 2048, 12288, 768),
+    (9, 2112, 16384, 256),
     (16, 768, 28672, 448),  # 64
     (31, 2048, 30000, 469),
     (48, 1536, 16384, 256),  # tiles of 64x64 from here on: wide for their rows
